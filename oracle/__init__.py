@@ -39,7 +39,7 @@ def build(reference: bool | None = None) -> None:
     """Compile the oracle (and oracle/_ref when the reference tree is present)."""
     subprocess.run(["make", "-s", "-C", str(ORACLE_DIR)], check=True)
     if reference is None:
-        reference = REFERENCE_ROOT.is_dir()
+        reference = (REFERENCE_ROOT / "native" / "src").is_dir()
     if reference:
         subprocess.run(["make", "-s", "-C", str(ORACLE_DIR), "ref"], check=True)
 
