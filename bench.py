@@ -1187,9 +1187,9 @@ def bench_boundary_fit(steps: int, cpu: bool):
 def bench_exact_svd(steps: int, cpu: bool):
     """The runtime's exact-SVD boundary initializer
     (exact_svd_boundary_launch_v1; runtime.py:335-389) on C1-style provider
-    heads: 32 heads (one layer slot) and 8,192, timed back to back.  The Jacobi
-    sweeps are a chain of 127 rounds per sweep behind one barrier each, so the
-    time is the chain, not HBM.  The CPU baseline is the reference's own call,
+    heads: 32 heads (one layer slot) and 8,192, timed back to back.  A head is
+    a chain of 126 reflections behind two barriers each, so the time is the
+    chain, not HBM.  The CPU baseline is the reference's own call,
     torch.linalg.svd in fp32 on the host, over the 32-head slot plus the
     residual and the quant stage (the oracle's encode), on the host's cores;
     the GPU's rank-4 product is checked against the float64 SVD on it."""
@@ -1218,7 +1218,7 @@ def bench_exact_svd(steps: int, cpu: bool):
     def call(n):
         return (stream, provider.data_ptr(), *(out[k].data_ptr() for k in out), n)
 
-    results = {"workload": "exact-SVD initializer (rank-4 truncated SVD by Jacobi + quant "
+    results = {"workload": "exact-SVD initializer (rank-4 truncated SVD + quant "
                            "stage) of C1-style provider heads"}
     for n in (32, heads):
         us = _time_back_to_back(fn, [call(n)], max(steps // 4, 2))

@@ -117,15 +117,15 @@ def exact_svd_boundary(provider: torch.Tensor, check: bool = True, residual=None
     (``GdnStateCodecRuntime._encode_dense_boundary``,
     ``src/gdn_state_codec/runtime.py:335-389``) for fp32 [...,128,128]
     provider heads ([value][key], the dense state transposed): the rank-4
-    truncated SVD of each dense head by one-sided Jacobi on the GPU, then the
-    quant-only encode of the fitted residual in the provider layout.
+    truncated SVD of each dense head on the GPU, then the quant-only encode of the fitted residual in the provider layout.
 
     Returns ``(codes, smoothing, scales, compensator_keys, compensator_values,
     residual, status)``: codes int8 [...,value,key], fp16 compensators
     [...,128,4] (keys = U*S, values = V), the fp32 residual [...,value,key]
     (``residual`` may name the buffer to write) and int32 ``status`` per head
     (0 ok, 1 non-finite input, 2 not converged within the sweep limit:
-    ``max_sweeps``, 1..30, default 30).  With ``check`` the call synchronizes
+    ``max_sweeps``, 1..30, default 30; below 30 every head takes Jacobi
+    sweeps, and only those can fail to converge).  With ``check`` the call synchronizes
     and raises ``ValueError`` for the first head with a nonzero status."""
     heads = _tiles(provider, torch.float32, "provider state")
     lead = tuple(provider.shape[:-2])

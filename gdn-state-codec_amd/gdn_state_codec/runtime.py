@@ -24,7 +24,7 @@ The interface is the reference runtime's: the method names
 ``project``, ``_slot``, ``invalidate``, ``decode_fallback_reason``,
 ``fall_back_to_native``, ``step``), the slot buffer names, the fallback reason
 keys, the two initializers (``quant_only`` and ``exact_svd``, the latter by
-the library's Jacobi SVD kernel instead of ``torch.linalg.svd``), and
+the library's own SVD kernels instead of ``torch.linalg.svd``), and
 ``RuntimeError`` for a violated contract or a non-zero launch status.  vLLM
 configuration parsing and the shadow observers are not part of this build;
 :class:`GdnStateCodecExperiment` carries only the fields read here.
@@ -421,7 +421,7 @@ class GdnStateCodecRuntime:
         """A new slot from one provider state [H][value][key] fp32 with the
         exact-SVD initializer (runtime.py:335-389): fp16 rank-4 compensators
         U*S and V of each dense head's truncated SVD, and the quant-only codes
-        of the residual, by one launch of the library's Jacobi SVD.  Raises
+        of the residual, by one call of the library's SVD.  Raises
         for a head with a non-finite value or one whose iteration did not
         converge."""
         boundary = self._provider_boundary(provider_dense)

@@ -120,19 +120,21 @@ int32_t statecentric_gdn_state_codec_quantize_boundary_launch_v1(
  * ([value][key], the dense [key][value] state transposed), replacing
  * GdnStateCodecRuntime._encode_dense_boundary(dense, "exact_svd")
  * (src/gdn_state_codec/runtime.py:335-389), which calls torch.linalg.svd:
- * the rank-4 truncated SVD of each dense head D = U S V^T by one-sided Jacobi,
+ * the rank-4 truncated SVD of each dense head D = U S V^T (the four largest
+ * eigenpairs of D^T D; one-sided Jacobi for heads whose leading singular values
+ * repeat),
  * compensator_keys fp16 [heads][128 key][4] = U[:, r] * S[r] and
  * compensator_values fp16 [heads][128 value][4] = V[:, r], r = 0..3 by
  * decreasing singular value; residual fp32 [heads][value][key] = the provider
  * tile minus the fp32 rank-4 product; then encode_launch_v4 of the residual in
  * the [value][key] layout (quantized [value][key], smoothing by key,
  * value_scales by value).  status[h] is 0; 1 when head h holds a
- * non-finite value (its outputs are then unspecified); or 2 when the Jacobi
+ * non-finite value (its outputs are then unspecified); or 2 when a Jacobi
  * iteration still rotated a pair in its last allowed sweep (30 here): the
  * outputs are then written from that sweep's rows, an unconverged fit the
  * caller should not take as the SVD.  The signs of each
- * (U, V) column pair are the iteration's own (an SVD fixes only their
- * product); the iteration runs in double, so the fp32 rank-4 product agrees
+ * (U, V) column pair are the solver's own (an SVD fixes only their
+ * product); it runs in double, so the fp32 rank-4 product agrees
  * with a float64 SVD to the fp32 rounding of the outputs (about 1e-7 of the
  * largest singular value).  1 <= heads <= 2^31-1.  No C-ABI counterpart in
  * the reference. */
@@ -143,7 +145,8 @@ int32_t statecentric_gdn_state_codec_exact_svd_boundary_launch_v1(
 
 /* exact_svd_boundary_launch_v1 with a caller-chosen limit of
  * 1 <= max_sweeps <= 30 Jacobi sweeps (status 1 for a limit outside it): a
- * head that has not converged within the limit gets status 2.  For callers
+ * head that has not converged within the limit gets status 2.  A limit below
+ * 30 runs the Jacobi iteration on every head; 30 is the entry point above.  For callers
  * that trade the fit's accuracy for time.  No counterpart in the reference. */
 int32_t statecentric_gdn_state_codec_exact_svd_boundary_sweeps_launch_v1(
     void* stream, const float* provider, float* residual, int8_t* quantized,

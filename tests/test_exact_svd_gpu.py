@@ -167,3 +167,60 @@ def test_sweep_limit_flags_unconverged_heads(device):
     for a, b in zip(full, default):
         assert a.tobytes() == b.tobytes()
     assert (full[-1] == 0).all()
+
+
+def mixed_heads(count, seed):
+    """Heads for both forms of the SVD in one batch: plain heads, a fourth
+    singular value just above and just below 2^-10 of the first (the direct
+    form's limit), ranks 1 to 5, and four equal leading singular values."""
+    g = np.random.default_rng(seed)
+    rest = np.linspace(0.9, 0.01, 124)
+    out = []
+    for i in range(count):
+        kind = i % 8
+        if kind < 2:
+            out.append(datagen.c1_heads(1, seed + i)[0])
+        elif kind < 4:
+            ratio = 2.0 ** -10 * (1.25 if kind == 2 else 0.8)
+            out.append(planted_head(seed + i, np.concatenate(
+                [[1.0, 0.5, 0.1, ratio], ratio * rest])))
+        elif kind < 7:
+            rank = 1 + (i // 8) % 5
+            out.append((g.standard_normal((128, rank))
+                        @ g.standard_normal((rank, 128))).astype(np.float32))
+        else:
+            out.append(planted_head(seed + i, np.concatenate([[3.0, 3.0, 3.0, 3.0], rest])))
+    return np.stack(out).astype(np.float32)
+
+
+@pytest.mark.parametrize("count", [1, 3, 40, 521])
+def test_direct_and_jacobi_forms_share_a_batch(device, count):
+    """Every head of a mixed batch, whichever form served it, holds the rank-4
+    product to the tolerance of the other tests; 521 heads leave more pending
+    heads than one Jacobi workgroup per CU, none of whose neighbours they may
+    disturb."""
+    dense = mixed_heads(count, 500)
+    print(f"exact SVD initializer, mixed batch of {count}", flush=True)
+    _, got = run(dense)
+    assert (got[6] == 0).all()
+    sample = sorted({*range(min(count, 40)), *range(0, count, 53), count - 1})
+    check_heads(dense[sample], [g[sample] for g in got],
+                rank_deficient=[n for n, h in enumerate(sample) if h % 8 in (4, 5, 6)])
+    # The sweep-limited entry point is Jacobi throughout: same product.
+    provider = torch.from_numpy(np.ascontiguousarray(dense.transpose(0, 2, 1))).cuda()
+    jacobi = [host(t) for t in codec.exact_svd_boundary(provider, max_sweeps=29)]
+    largest = np.abs(dense).max(axis=(1, 2)) * 128  # at least sigma_1
+    apart = np.abs(got[5].astype(np.float64) - jacobi[5]).max(axis=(1, 2))
+    assert (apart <= 2 * FIT_TOLERANCE * largest).all()
+
+
+def test_residual_may_overwrite_the_provider_state(device):
+    """residual naming the provider buffer itself: each cell is read for the
+    last time by the thread that writes it."""
+    dense = mixed_heads(9, 700)
+    provider = torch.from_numpy(np.ascontiguousarray(dense.transpose(0, 2, 1))).cuda()
+    apart = [host(t) for t in codec.exact_svd_boundary(provider)]
+    inside = [host(t) for t in codec.exact_svd_boundary(provider, residual=provider)]
+    print("exact SVD initializer in place", flush=True)
+    for a, b in zip(apart, inside):
+        assert a.tobytes() == b.tobytes()
