@@ -31,6 +31,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "codec_math.h"
 #include "gdn_state_codec_window.h"
 #include "lane_exchange.h"
 #include "launch.h"
@@ -89,14 +90,6 @@ __device__ __forceinline__ int chain_round(float value) {
   r = r > 127.0f ? 127.0f : r;
   r = r < -127.0f ? -127.0f : r;
   return static_cast<int>(r);
-}
-
-// window_boundary.cpp:17-23 / encoded_projection.cpp:36-42.
-__device__ __forceinline__ float chain_newton_sqrt(float value) {
-  float estimate = value > 1.0f ? value : 1.0f;
-#pragma unroll 1
-  for (int i = 0; i < 20; ++i) estimate = 0.5f * (estimate + value / estimate);
-  return estimate;
 }
 
 // prepare_int8_vector of the current vector on input side `side`
@@ -202,7 +195,7 @@ __device__ void chain_finish(ChainShared& sh, int in_side, uint32_t ranks, int l
     squared_norm += v.z * v.z;
     squared_norm += v.w * v.w;
   }
-  const float inverse = squared_norm > 1.0e-20f ? 1.0f / chain_newton_sqrt(squared_norm) : 0.0f;
+  const float inverse = squared_norm > 1.0e-20f ? 1.0f / newton_sqrt(squared_norm) : 0.0f;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int row = lane + h * kChainLanes;

@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "codec_math.h"
 #include "gdn_state_codec_window.h"
 #include "launch.h"
 #include "window_common.h"
@@ -57,14 +58,6 @@ struct RankArgs {
   uint32_t ranks;       // finish: fitted ranks (0..4); commit: the rank committed (0..3)
   uint32_t transpose;   // finish only
 };
-
-// window_boundary.cpp:17-23 / encoded_projection.cpp:36-42.
-__device__ __forceinline__ float newton_sqrt(float value) {
-  float estimate = value > 1.0f ? value : 1.0f;
-#pragma unroll 1
-  for (int i = 0; i < 20; ++i) estimate = 0.5f * (estimate + value / estimate);
-  return estimate;
-}
 
 __device__ __forceinline__ float readlane(float value, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(value), lane));

@@ -99,14 +99,6 @@ struct PowerShared {
 };
 static_assert(workgroups_by_lds(sizeof(PowerShared)) >= 5, "five workgroups per CU");
 
-// window_boundary.cpp:17-23.
-__device__ __forceinline__ float newton_sqrt(float value) {
-  float estimate = value > 1.0f ? value : 1.0f;
-#pragma unroll 1
-  for (int i = 0; i < 20; ++i) estimate = 0.5f * (estimate + value / estimate);
-  return estimate;
-}
-
 __device__ __forceinline__ float h2f(uint16_t h) { return half_bits_to_float(h); }
 
 // code / 127 by the two-part division (div_by_127, exact for every integer in

@@ -334,6 +334,31 @@ void check_wide_lift() {
   fprintf(stderr, "fallbacks %llu\n", static_cast<unsigned long long>(fallbacks.load()));
 }
 
+// newton_sqrt against the 20 steps themselves: every 61st float of each exponent
+// from 2^-34 to 2^33 (both forms), and the floats around the form's limits.
+void check_newton() {
+  const auto steps = [](float value) {
+    float estimate = value > 1.0f ? value : 1.0f;
+    for (int i = 0; i < 20; ++i) estimate = 0.5f * (estimate + value / estimate);
+    return estimate;
+  };
+  const auto check = [&](uint32_t bits) {
+    float value;
+    memcpy(&value, &bits, 4);
+    const float got = gdn::newton_sqrt(value), want = steps(value);
+    ++checked;
+    if (memcmp(&got, &want, 4) != 0) ++failures;
+  };
+  for (uint32_t exponent = 127 - 34; exponent <= 127 + 33; ++exponent) {
+    for (uint32_t m = 0; m < (1u << 23); m += 61) check((exponent << 23) | m);
+  }
+  for (int exponent : {-32, 0, 32}) {
+    const uint32_t edge = static_cast<uint32_t>(127 + exponent) << 23;
+    for (uint32_t bits = edge - 4096; bits < edge + 4096; ++bits) check(bits);
+  }
+  for (uint32_t bits : {0u, 0x00800000u, 0x7F7FFFFFu, 0x7F800000u}) check(bits);
+}
+
 void check_order_grid(uint64_t blocks) {
   std::vector<uint8_t> seen(blocks, 0);
   bool ok = true;
@@ -378,6 +403,8 @@ int main(int argc, char** argv) {
   } else if (strcmp(argv[1], "lift_refit") == 0) {
     refit_rounding = true;
     check_lift();
+  } else if (strcmp(argv[1], "newton") == 0) {
+    check_newton();
   } else if (strcmp(argv[1], "order") == 0) {
     check_order();
   } else {

@@ -102,6 +102,15 @@ def test_bf16_direct_lift_matches_lround_wherever_its_margin_admits_it(checker):
     assert checked > 400_000_000 and failures == 0 and rc == 0
 
 
+def test_newton_root_equals_its_twenty_steps(checker):
+    """newton_sqrt (one step from the correctly rounded root over [2^-32, 2^32),
+    the 20 steps outside) against the reference's 20 steps, bit for bit: every
+    61st float of 68 exponents, the limits' neighbourhoods, 0, the smallest and
+    largest normal and infinity."""
+    rc, checked, failures = _run(checker, "newton")
+    assert checked == 68 * 137519 + 3 * 8192 + 4 and failures == 0 and rc == 0
+
+
 def test_xcd_contiguous_order_is_a_bijection(checker):
     """The streaming kernels' workgroup -> tile order (csrc/work_order.h) visits
     every tile exactly once for every grid size up to 4,096 and the bench's."""
