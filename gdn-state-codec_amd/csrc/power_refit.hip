@@ -11,16 +11,26 @@
 // round-half-away codes, and the window is cleared.
 //
 // Every dot product of the reference is a sequential fp32 sum; this kernel
-// keeps each one on a single thread in the reference's order (outputs of the
-// operator in parallel, one row or column per thread; projections and norms
-// on single threads, broadcast through LDS), so the result is bit-identical to
-// the CPU statement of the reference kernel.  One 128-thread workgroup per
-// state, operands staged in LDS: the codes at a 132-byte row stride so both
-// the row walk and the column walk are free of bank conflicts, compensators
-// and records as fp16 bits (31,408 bytes: 25 of the CU's 1,280-byte LDS
-// granules, five workgroups per CU).  The fitted residual is evaluated once
-// per cell, one key row per thread held in registers for the smoothing, scale
-// and code passes, and written once to the workspace.
+// keeps each one on a single thread in the reference's order, so the result is
+// bit-identical to the CPU statement of the reference kernel.
+//
+// One workgroup per state, in two forms (kSplitStates says where the line
+// between them lies):
+//   split, 256 threads: threads 0..127 own the key rows and 128..255 the value
+//     columns, each with its line's 128 boundary values code / 127 * s * scale
+//     in VGPRs (168, so three states per CU).  An operator application sums on
+//     the side that owns its outputs, while a wavefront of the other side forms
+//     the 24 projections of the compensators, records and fitted ranks.
+//   whole, 128 threads: thread t owns row t and column t, with their codes in
+//     64 VGPRs and the values formed again in every application (eight
+//     instructions a value instead of three), which leaves five states per CU
+//     (31,920 bytes of LDS each).
+// In both one wavefront sums a vector's squared norm and normalizes it.  The
+// chains of one state bound the kernel when there are few states (per
+// application 128 products and adds, 24 more terms and 128 adds), VALU issue
+// when there are many.  The fitted residual is evaluated once per cell, one key
+// row per thread held in registers for the smoothing, scale and code passes,
+// and written once to the workspace.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -37,9 +47,18 @@
 namespace gdn {
 namespace {
 
-constexpr int kThreads = 128;
+constexpr int kThreads = 128;       // one thread per row (and column)
+constexpr int kSplitThreads = 256;  // one thread per row, one per column
 constexpr int kCodeStride = kDim + 4;
 constexpr float kBoundaryFloor = 1.0e-8f;
+// The split form up to what runs at once with three states per CU: one state's
+// latency is what counts there.  4 iterations, split / whole form (and the
+// form before both, which formed each value from LDS with a rolled loop, a
+// thread for row and column), us: 32 states 158 / 231 (324), 256 states 168 /
+// 241 (298), 768 states 223 / 285 (320), 1,024 states 362 / 306 (325), 8,192
+// states 2,311 / 2,077 (2,288).  At 1,536 and 2,304 states the split form's
+// rounds come out full and it is ahead by 16% and 2%, at 1,280 behind by 7%.
+constexpr uint32_t kSplitStates = 768;
 
 // f(std::integral_constant<int, c>) for c = 0 .. kDim - 1, expanded at compile
 // time: a body that indexes a register array by c keeps the array in VGPRs,
@@ -73,7 +92,7 @@ struct PowerArgs {
 
 // Compensators and records are fp16 values (the fitted ranks are rounded to
 // fp16 when formed), so they are kept as fp16 bits and widened exactly when
-// read: 31,408 bytes, five workgroups per CU.
+// read: 31,920 bytes, five workgroups per CU.
 struct PowerShared {
   int8_t code[kDim * kCodeStride];  // [value column][key row]
   alignas(8) uint16_t ck[kDim * kRank];
@@ -87,19 +106,16 @@ struct PowerShared {
   alignas(16) uint16_t rk[kDim * kWindow];
   alignas(16) uint16_t rc[kDim * kWindow];
   float smoothing[kDim], scales[kDim];
-  union {
-    float left[kDim];            // power iteration
-    float next_smoothing[kDim];  // re-encoding, after the iteration
-  };
-  float right[kDim];
-  float old_projection[kRank], fitted_projection[kRank], record_projection[kWindow];
-  float record_suffix[kWindow];
-  float scalar;  // norm inverse / singular value broadcast
-  int flag;
+  alignas(16) float left[kDim];
+  alignas(16) float right[kDim];
+  alignas(16) float square[kDim];  // of the vector just formed, for its norm
+  // The projections of an application: old ranks, fitted ranks, records.
+  alignas(16) float projection[2 * kRank + kWindow];
+  alignas(16) float record_suffix[kWindow];
+  float scalar;  // the singular value
+  int flag;      // whether the vector could be normalized
 };
 static_assert(workgroups_by_lds(sizeof(PowerShared)) >= 5, "five workgroups per CU");
-
-__device__ __forceinline__ float h2f(uint16_t h) { return half_bits_to_float(h); }
 
 // code / 127 by the two-part division (div_by_127, exact for every integer in
 // [-128, 127]): two VALU instructions, where a table of the 256 quotients
@@ -108,104 +124,168 @@ __device__ __forceinline__ float code_value_arith(int8_t code) {
   return div_by_127(static_cast<float>(code));
 }
 
-// Normalize (:25-37) of v; returns whether the norm was usable.  The squared
-// norm is one sequential sum on thread 0.
-__device__ bool normalize(PowerShared& sh, float* v, int t) {
-  if (t == 0) {
-    float squared = 0.0f;
-    struct Group {
-      float x[16];
-    };
-    pipelined<kDim / 16, Group>(
-        [&](auto g, Group& r) { unrolled<16>([&](auto i) { r.x[i] = v[16 * decltype(g)::value + i]; }); },
-        [&](auto, const Group& r) { unrolled<16>([&](auto i) { squared += r.x[i] * r.x[i]; }); });
-    sh.flag = squared <= 1.0e-20f ? 0 : 1;
-    sh.scalar = sh.flag ? 1.0f / newton_sqrt(squared) : 0.0f;
-  }
-  __syncthreads();
-  const bool ok = sh.flag != 0;
-  if (ok) v[t] *= sh.scalar;
-  __syncthreads();
-  return ok;
+// The sequential sum of sh.square, evaluated identically by every lane.
+__device__ __forceinline__ float squared_norm(const PowerShared& sh) {
+  float squared = 0.0f;
+  struct Group {
+    float x[16];
+  };
+  pipelined<kDim / 16, Group>(
+      [&](auto g, Group& r) {
+        unrolled<4>([&](auto q) {
+          *reinterpret_cast<float4*>(r.x + 4 * decltype(q)::value) =
+              *reinterpret_cast<const float4*>(sh.square + 16 * decltype(g)::value +
+                                               4 * decltype(q)::value);
+        });
+      },
+      [&](auto, const Group& r) { unrolled<16>([&](auto i) { squared += r.x[i]; }); });
+  return squared;
 }
 
-// Projections of an apply (old compensator side, records, fitted ranks): one
-// sequential sum per thread in the reference's loop order.  Wavefront 0 runs
-// the compensator sides (lanes 0..3 the old ranks, lanes 4..7 the fitted
-// ones: the same loop over a per-lane basis, so no branch divergence) while
-// wavefront 1 runs the 16 record sides (its lanes 0..15).
-__device__ void projections(PowerShared& sh, const float* vector, const uint16_t* old_basis,
-                            const uint16_t* record_basis, const uint16_t* fitted_basis,
-                            int fitted, int t) {
-  if (t < 2 * kRank) {
-    const int r = t & (kRank - 1);
-    const bool is_fitted = t >= kRank;
-    if (!is_fitted || r < fitted) {
-      const uint16_t* basis = is_fitted ? fitted_basis : old_basis;
-      float acc = 0.0f;
-      for (int i = 0; i < kDim; ++i) acc += h2f(basis[i * kRank + r]) * vector[i];
-      if (is_fitted) {
-        sh.fitted_projection[r] = acc;
-      } else {
-        sh.old_projection[r] = acc;
-      }
+// Normalize (:25-37) of `vector` by one wavefront; a vector whose norm is not
+// usable stays as it is.
+__device__ __forceinline__ void normalize(PowerShared& sh, float* vector, int lane) {
+  const float squared = squared_norm(sh);
+  const bool ok = !(squared <= 1.0e-20f);
+  if (ok) {
+    const float inverse = 1.0f / newton_sqrt(squared);
+    vector[lane] *= inverse;
+    vector[64 + lane] *= inverse;
+  }
+  if (lane == 0) sh.flag = ok ? 1 : 0;
+}
+
+// The projections of an application (old compensator side, fitted ranks,
+// records) by one wavefront: one sequential sum per lane in the reference's
+// loop order, a product of an fp16 and an fp32 value being one v_fma_mix_f32
+// (adding -0 changes nothing).  Ranks not fitted yet are zero in LDS and their
+// sums are not used.
+__device__ __forceinline__ void projections(PowerShared& sh, const float* vector,
+                                            const uint16_t* old_basis,
+                                            const uint16_t* record_basis,
+                                            const uint16_t* fitted_basis, int lane) {
+  if (lane >= 2 * kRank + kWindow) return;
+  const uint16_t* const basis = lane < kRank ? old_basis + lane
+                                : lane < 2 * kRank ? fitted_basis + (lane - kRank)
+                                                   : record_basis + (lane - 2 * kRank);
+  const int stride = lane < 2 * kRank ? kRank : kWindow;
+  const float neg_zero = opaque_negative_zero();
+  float acc = 0.0f;
+  struct Group {
+    float x[8];
+    uint16_t b[8];
+  };
+  Group now, ahead;
+  const auto load = [&](int i, Group& g) {
+    *reinterpret_cast<float4*>(g.x) = *reinterpret_cast<const float4*>(vector + i);
+    *reinterpret_cast<float4*>(g.x + 4) = *reinterpret_cast<const float4*>(vector + i + 4);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g.b[e] = basis[(i + e) * stride];
+  };
+  load(0, now);
+#pragma unroll 2
+  for (int i = 0; i < kDim; i += 8) {
+    load((i + 8) & (kDim - 1), ahead);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      acc += __builtin_fmaf(half_bits_to_float(now.b[e]), now.x[e], neg_zero);
     }
-  } else if (t >= 64 && t < 64 + kWindow) {
-    const int j = t - 64;
-    float acc = 0.0f;
-    for (int i = 0; i < kDim; ++i) acc += h2f(record_basis[i * kWindow + j]) * vector[i];
-    sh.record_projection[j] = acc;
+    now = ahead;
   }
-  __syncthreads();
+  sh.projection[lane] = acc;
 }
 
-// ApplyRight (:113-166): output[row] = R^T-free form R * vector over columns.
-__device__ void apply_right(PowerShared& sh, const float* vector, float* output, float bs,
-                            int fitted, int t) {
-  projections(sh, vector, sh.cv, sh.rc, sh.nv, fitted, t);
-  const int row = t;
+// The sum of an application's boundary part (:113-142, :168-197) over a line's
+// values: value = ((code / 127 * s) * scale) * vector * bs, in order.
+__device__ __forceinline__ float line_sum(const float (&cell)[kDim], const float* vector,
+                                          float bs) {
   float value = 0.0f;
-  const float s = sh.smoothing[row];
-  for (int column = 0; column < kDim; ++column) {
-    value += code_value_arith(sh.code[column * kCodeStride + row]) * s * sh.scales[column] *
-             vector[column] * bs;
-  }
-  for (int r = 0; r < kRank; ++r) value += h2f(sh.ck[row * kRank + r]) * sh.old_projection[r] * bs;
-  for (int j = 0; j < kWindow; ++j) {
-    value += h2f(sh.rk[row * kWindow + j]) * sh.record_projection[j] * sh.record_suffix[j];
-  }
-  for (int r = 0; r < fitted; ++r) value -= h2f(sh.nk[row * kRank + r]) * sh.fitted_projection[r];
-  __syncthreads();  // every thread has read `vector` before it may be overwritten
-  output[row] = value;
-  __syncthreads();
+  struct Group {
+    float x[8];
+  };
+  pipelined<kDim / 8, Group>(
+      [&](auto g, Group& r) {
+        constexpr int first = 8 * decltype(g)::value;
+        *reinterpret_cast<float4*>(r.x) = *reinterpret_cast<const float4*>(vector + first);
+        *reinterpret_cast<float4*>(r.x + 4) = *reinterpret_cast<const float4*>(vector + first + 4);
+      },
+      [&](auto g, const Group& r) {
+        unrolled<8>([&](auto i) {
+          value += cell[8 * decltype(g)::value + decltype(i)::value] * r.x[i] * bs;
+        });
+      });
+  return value;
 }
 
-// ApplyTranspose (:168-221): output[column] = R^T * vector over rows.
-__device__ void apply_transpose(PowerShared& sh, const float* vector, float* output, float bs,
-                                int fitted, int t) {
-  projections(sh, vector, sh.ck, sh.rk, sh.nk, fitted, t);
-  const int column = t;
+// The same sum with the line's codes packed four to a word in place of its
+// values; `own` is the line's factor, `across` the other axis' factors, and
+// `rows` tells which of the two is the smoothing (code / 127 * s * scale).
+template <bool kRows>
+__device__ __forceinline__ float code_sum(const uint32_t (&codes)[kDim / 4], const float* vector,
+                                          const float* across, float own, float bs) {
   float value = 0.0f;
-  const float scale = sh.scales[column];
-  const int8_t* code = sh.code + column * kCodeStride;
-  for (int row = 0; row < kDim; ++row) {
-    value += code_value_arith(code[row]) * sh.smoothing[row] * scale * vector[row] * bs;
-  }
-  for (int r = 0; r < kRank; ++r) value += h2f(sh.cv[column * kRank + r]) * sh.old_projection[r] * bs;
-  for (int j = 0; j < kWindow; ++j) {
-    value += h2f(sh.rc[column * kWindow + j]) * sh.record_projection[j] * sh.record_suffix[j];
-  }
-  for (int r = 0; r < fitted; ++r) value -= h2f(sh.nv[column * kRank + r]) * sh.fitted_projection[r];
-  __syncthreads();
-  output[column] = value;
-  __syncthreads();
+  struct Group {
+    float x[4], f[4];
+  };
+  pipelined<kDim / 4, Group>(
+      [&](auto g, Group& r) {
+        constexpr int first = 4 * decltype(g)::value;
+        *reinterpret_cast<float4*>(r.x) = *reinterpret_cast<const float4*>(vector + first);
+        *reinterpret_cast<float4*>(r.f) = *reinterpret_cast<const float4*>(across + first);
+      },
+      [&](auto g, const Group& r) {
+        // Opaque, so that the widened codes are not formed once for all
+        // applications and held (spilled) between them.
+        uint32_t word = codes[decltype(g)::value];
+        asm volatile("" : "+v"(word));
+        unrolled<4>([&](auto i) {
+          constexpr int b = decltype(i)::value;
+          const float code = code_value_arith(static_cast<int8_t>(word >> (8 * b)));
+          const float cell = kRows ? code * own * r.f[b] : code * r.f[b] * own;
+          value += cell * r.x[b] * bs;
+        });
+      });
+  return value;
 }
 
-// The re-encode of R minus the fit, for the 128 threads of a workgroup whose
-// LDS holds the state (codes [value column][key row] at kCodeStride, the old
+// The rest of an application for line `line` (:143-165, :198-220): the old
+// compensators, the records, less the fitted ranks.
+__device__ __forceinline__ float line_terms(const PowerShared& sh, float value, int line,
+                                            const uint16_t* old_basis,
+                                            const uint16_t* record_basis,
+                                            const uint16_t* fitted_basis, float bs, int fitted) {
+  const float neg_zero = opaque_negative_zero();
+  const auto half = [](uint32_t pair, int i) { return i & 1 ? pair >> 16 : pair; };
+  const auto times = [&](uint32_t bits, float x) {
+    return __builtin_fmaf(half_bits_to_float(bits), x, neg_zero);
+  };
+  const uint2 old2 = *reinterpret_cast<const uint2*>(old_basis + line * kRank);
+  const uint2 new2 = *reinterpret_cast<const uint2*>(fitted_basis + line * kRank);
+  const uint4 r0 = reinterpret_cast<const uint4*>(record_basis + line * kWindow)[0];
+  const uint4 r1 = reinterpret_cast<const uint4*>(record_basis + line * kWindow)[1];
+  const uint32_t olds[2] = {old2.x, old2.y}, news[2] = {new2.x, new2.y};
+  const uint32_t records[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+  for (int r = 0; r < kRank; ++r) value += times(half(olds[r / 2], r), sh.projection[r]) * bs;
+#pragma unroll
+  for (int j = 0; j < kWindow; ++j) {
+    value += times(half(records[j / 2], j), sh.projection[2 * kRank + j]) * sh.record_suffix[j];
+  }
+#pragma unroll
+  for (int r = 0; r < kRank; ++r) {
+    if (r < fitted) value -= times(half(news[r / 2], r), sh.projection[kRank + r]);
+  }
+  return value;
+}
+
+// The re-encode of R minus the fit, for 128 threads of a workgroup (those with
+// `active`, whole wavefronts; the others only meet its barriers) whose LDS
+// holds the state (codes [value column][key row] at kCodeStride, the old
 // and fitted compensators ck / cv / nk / nv [dim][rank], the records rk / rc
-// [dim][record], smoothing, scales and record suffixes):
-// thread t owns key row t, whose 128 fitted cells stay in registers through
+// [dim][record], smoothing, scales and record suffixes).  With kFromCodes the
+// boundary values come from the codes in LDS, else cell[] holds them already.
+// Thread t owns key row t, whose 128 fitted cells stay in registers through
 // the smoothing, scale and code passes.  Writes the fitted residual to
 // workspace [key row][value column], next_smoothing[key], next_scales[value],
 // and hands every code of row t to sink(integral_constant column, code).  Each
@@ -214,17 +294,18 @@ __device__ void apply_transpose(PowerShared& sh, const float* vector, float* out
 // order.  The column loops are unrolled at compile time (each_column) so that
 // cell[] is only ever indexed by constants and lives in VGPRs.  Uses sh.left
 // and sh.right as scratch for the column maxima.
-template <typename Sink>
-__device__ __forceinline__ void reencode_rows(PowerShared& sh, float bs, int t, float* workspace,
+template <bool kFromCodes, typename Sink>
+__device__ __forceinline__ void reencode_rows(PowerShared& sh, float (&cell)[kDim], bool active,
+                                              float bs, int t, float* workspace,
                                               float* next_smoothing, float* next_scales,
                                               Sink&& sink) {
   const int row = t;
-  float cell[kDim];
+  if (active) {
   {
     // The row's operands stay as fp16 pairs (widened where used) and the
     // window suffix products, the same for every thread, in scalar
     // registers, leaving the vector registers to the cells.
-    const float s = sh.smoothing[row];
+    [[maybe_unused]] const float s = sh.smoothing[row];
     uint32_t ck2[kRank / 2], nk2[kRank / 2], rk2[kWindow / 2];
     float suffix[kWindow];
 #pragma unroll
@@ -247,15 +328,17 @@ __device__ __forceinline__ void reencode_rows(PowerShared& sh, float bs, int t, 
     // A column's LDS operands; the next column's are read while this one's
     // cell is evaluated, so their latency overlaps the arithmetic.
     struct Operands {
-      int code;
-      float scale;
+      int code;     // with kFromCodes
+      float scale;  // with kFromCodes
       uint2 cv, nv;
       uint4 r0, r1;
     };
     const auto fetch = [&](int column) {
       Operands o;
-      o.code = sh.code[column * kCodeStride + row];
-      o.scale = sh.scales[column];
+      if constexpr (kFromCodes) {
+        o.code = sh.code[column * kCodeStride + row];
+        o.scale = sh.scales[column];
+      }
       o.cv = *reinterpret_cast<const uint2*>(sh.cv + column * kRank);
       o.nv = *reinterpret_cast<const uint2*>(sh.nv + column * kRank);
       const uint4* const rc4 = reinterpret_cast<const uint4*>(sh.rc + column * kWindow);
@@ -276,7 +359,12 @@ __device__ __forceinline__ void reencode_rows(PowerShared& sh, float bs, int t, 
       // Issued here, ahead of this column's arithmetic, not sunk to its end.
       __builtin_amdgcn_sched_barrier(0);
       // code / 127 by the two-part division (exact for every integer code).
-      float value = code_value_arith(static_cast<int8_t>(o.code)) * s * o.scale * bs;
+      float value;
+      if constexpr (kFromCodes) {
+        value = code_value_arith(static_cast<int8_t>(o.code)) * s * o.scale * bs;
+      } else {
+        value = cell[column] * bs;
+      }
       const uint32_t cvp[kRank / 2] = {o.cv.x, o.cv.y}, nvp[kRank / 2] = {o.nv.x, o.nv.y};
 #pragma unroll
       for (int r = 0; r < kRank; ++r) {
@@ -348,8 +436,9 @@ __device__ __forceinline__ void reencode_rows(PowerShared& sh, float bs, int t, 
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  }  // active
   __syncthreads();  // both wavefronts' column maxima; every cell has been evaluated
-  {
+  if (active) {
     // Thread t's own slots: no other thread reads them before the barrier.
     const float maximum = fmaxf(sh.left[t], sh.right[t]);
     next_scales[t] = maximum;
@@ -371,6 +460,7 @@ __device__ __forceinline__ void reencode_rows(PowerShared& sh, float bs, int t, 
   // (the certificate of codec_math.h; |m| <= maximum since the maximum is
   // over these same m).  The other cells, NaN and infinite ones among them,
   // take the reference's expression.
+  if (!active) return;
   each_column([&](auto c) {
     constexpr int column = decltype(c)::value;
     const float m = cell[column];
@@ -391,34 +481,41 @@ __device__ __forceinline__ void reencode_rows(PowerShared& sh, float bs, int t, 
   });
 }
 
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) void power_refit_kernel(PowerArgs a) {
+template <bool kSplit>
+__global__ __launch_bounds__(kSplit ? kSplitThreads : kThreads) __attribute__((amdgpu_waves_per_eu(3))) void power_refit_kernel(PowerArgs a) {
+  constexpr int kFitThreads = kSplit ? kSplitThreads : kThreads;
   extern __shared__ __align__(16) unsigned char dynamic[];
   PowerShared& sh = *reinterpret_cast<PowerShared*>(dynamic);
   const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int line = t & (kDim - 1);   // the thread's row or column
+  const bool rows = !kSplit || wave < 2;     // it owns a key row,
+  const bool columns = !kSplit || wave > 1;  // a value column
   const uint64_t state = blockIdx.x;
   if (a.positions[state * kPositionStride] != static_cast<uint32_t>(kWindow)) return;  // uniform
   const uint64_t vb = state * kDim;
   const uint64_t rb = state * kWindow;
 
   // ---- stage the state in LDS -----------------------------------------------
-  for (int i = t; i < kTile / 4; i += kThreads) {
+  for (int i = t; i < kTile / 4; i += kFitThreads) {
     const uint32_t w = reinterpret_cast<const uint32_t*>(a.residual + state * kTile)[i];
     const int column = (4 * i) / kDim, row = (4 * i) % kDim;
     *reinterpret_cast<uint32_t*>(&sh.code[column * kCodeStride + row]) = w;
   }
-  for (int i = t; i < kDim * kRank; i += kThreads) {
+  for (int i = t; i < kDim * kRank; i += kFitThreads) {
     sh.ck[i] = a.comp_keys[vb * kRank + i];
     sh.cv[i] = a.comp_values[vb * kRank + i];
     sh.nk[i] = 0u;
     sh.nv[i] = 0u;
   }
-  for (int i = t; i < kWindow * kDim; i += kThreads) {
+  for (int i = t; i < kWindow * kDim; i += kFitThreads) {
     const int j = i / kDim, dimension = i % kDim;
     sh.rk[dimension * kWindow + j] = a.record_keys[rb * kDim + i];
     sh.rc[dimension * kWindow + j] = a.record_corrections[rb * kDim + i];
   }
-  sh.smoothing[t] = (a.smoothing + vb)[t];
-  sh.scales[t] = (a.scales + vb)[t];
+  if (rows) sh.smoothing[line] = (a.smoothing + vb)[line];
+  if (columns) sh.scales[line] = (a.scales + vb)[line];
   // BuildSuffix (:102-111), computed identically by every thread.
   float bs = 1.0f;
   for (int j = kWindow - 1; j >= 0; --j) {
@@ -429,45 +526,120 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
   bs = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(bs)));
   __syncthreads();
 
+  // ---- the lines' boundary values (code / 127 * s * scale), or their codes ----
+  float cell[kDim];
+  uint32_t row_codes[kDim / 4], column_codes[kDim / 4];
+  if constexpr (!kSplit) {
+    each_column([&](auto c) {
+      constexpr int column = decltype(c)::value;
+      const uint32_t code = static_cast<uint8_t>(sh.code[column * kCodeStride + line]);
+      row_codes[column / 4] =
+          column % 4 == 0 ? code : row_codes[column / 4] | (code << (8 * (column % 4)));
+      if constexpr (column % 4 == 0) {
+        column_codes[column / 4] =
+            *reinterpret_cast<const uint32_t*>(&sh.code[line * kCodeStride + column]);
+      }
+    });
+  } else if (rows) {
+    const float s = sh.smoothing[line];
+    each_column([&](auto c) {
+      constexpr int column = decltype(c)::value;
+      cell[column] = code_value_arith(sh.code[column * kCodeStride + line]) * s * sh.scales[column];
+      if constexpr (column % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+    });
+  } else {
+    const float scale = sh.scales[line];
+    each_column([&](auto c) {
+      constexpr int row = decltype(c)::value;
+      cell[row] = code_value_arith(sh.code[line * kCodeStride + row]) * sh.smoothing[row] * scale;
+      if constexpr (row % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+
   // ---- deflated power iteration ---------------------------------------------
-  for (int rank = 0; rank < kRank; ++rank) {
-    sh.right[t] = static_cast<float>(static_cast<int>(((rank + 1) * (t + 3)) % 17) - 8);
-    __syncthreads();
-    (void)normalize(sh, sh.right, t);
-    for (uint32_t it = 0; it < a.power_iterations; ++it) {
-      apply_right(sh, sh.right, sh.left, bs, rank, t);
-      if (!normalize(sh, sh.left, t)) break;
-      apply_transpose(sh, sh.left, sh.right, bs, rank, t);
-      if (!normalize(sh, sh.right, t)) break;
+  // ApplyRight (:113-166, forward: right vector in, one row's sum out) and
+  // ApplyTranspose (:168-221): the sums on the side that owns the outputs, the
+  // projections in a wavefront of the other side; the result and its squares
+  // are published by the last barrier.
+  const auto apply = [&](bool forward, int fitted) {
+    const float* const in = forward ? sh.right : sh.left;
+    float* const out = forward ? sh.left : sh.right;
+    const bool own = forward ? rows : columns;
+    float value = 0.0f;
+    // Split: a wavefront of the other side, while this one sums.
+    if (wave == (kSplit ? (forward ? 2 : 0) : (forward ? 1 : 0))) {
+      projections(sh, in, forward ? sh.cv : sh.ck, forward ? sh.rc : sh.rk,
+                  forward ? sh.nv : sh.nk, lane);
     }
-    apply_right(sh, sh.right, sh.left, bs, rank, t);
-    if (t == 0) {
-      float squared = 0.0f;
-      for (int i = 0; i < kDim; ++i) squared += sh.left[i] * sh.left[i];
-      sh.scalar = newton_sqrt(squared);
+    if (own) {
+      if constexpr (kSplit) {
+        value = line_sum(cell, in, bs);
+      } else if (forward) {
+        value = code_sum<true>(row_codes, in, sh.scales, sh.smoothing[line], bs);
+      } else {
+        value = code_sum<false>(column_codes, in, sh.smoothing, sh.scales[line], bs);
+      }
+    }
+    __syncthreads();
+    if (own) {
+      value = line_terms(sh, value, line, forward ? sh.ck : sh.cv, forward ? sh.rk : sh.rc,
+                         forward ? sh.nk : sh.nv, bs, fitted);
+      out[line] = value;
+      sh.square[line] = value * value;
+    }
+    __syncthreads();
+  };
+  const auto normalized = [&](float* vector) {
+    if (wave == 1) normalize(sh, vector, lane);
+    __syncthreads();
+    return sh.flag != 0;  // uniform
+  };
+  for (int rank = 0; rank < kRank; ++rank) {
+    if (rows) {
+      const float v = static_cast<float>(static_cast<int>(((rank + 1) * (line + 3)) % 17) - 8);
+      sh.right[line] = v;
+      sh.square[line] = v * v;
+    }
+    __syncthreads();
+    (void)normalized(sh.right);
+    for (uint32_t it = 0; it < a.power_iterations; ++it) {
+      apply(true, rank);
+      if (!normalized(sh.left)) break;
+      apply(false, rank);
+      if (!normalized(sh.right)) break;
+    }
+    apply(true, rank);
+    if (wave == 1) {
+      const float singular = newton_sqrt(squared_norm(sh));
+      if (lane == 0) sh.scalar = singular;
     }
     __syncthreads();
     const float singular = sh.scalar;
     if (singular > 1.0e-20f) {
       const float inverse = 1.0f / singular;
-      sh.nk[t * kRank + rank] = static_cast<uint16_t>(float_to_half_bits(sh.left[t] * inverse * singular));
-      sh.nv[t * kRank + rank] = static_cast<uint16_t>(float_to_half_bits(sh.right[t]));
+      if (rows) {
+        sh.nk[line * kRank + rank] =
+            static_cast<uint16_t>(float_to_half_bits(sh.left[line] * inverse * singular));
+      }
+      if (columns) {
+        sh.nv[line * kRank + rank] = static_cast<uint16_t>(float_to_half_bits(sh.right[line]));
+      }
     }
     __syncthreads();
   }
 
   // ---- R minus the fit, re-encoded; codes staged in the code area ------------
   // The workspace is written once and never read back.
-  reencode_rows(sh, bs, t, a.workspace + state * kTile, a.next_smoothing + vb, a.next_scales + vb,
-                [&](auto c, int8_t code) {
-                  sh.code[decltype(c)::value * kCodeStride + t] = code;
-                });
+  reencode_rows<!kSplit>(sh, cell, rows, bs, line, a.workspace + state * kTile,
+                       a.next_smoothing + vb, a.next_scales + vb, [&](auto c, int8_t code) {
+                         sh.code[decltype(c)::value * kCodeStride + line] = code;
+                       });
   __syncthreads();
-  // next_residual [value column][key row]: each round of 16 columns, eight
-  // lanes write one whole 128-byte column.
+  // next_residual [value column][key row], eight lanes to a whole 128-byte
+  // column.
 #pragma unroll
-  for (int round = 0; round < kDim / 16; ++round) {
-    const int column = 16 * round + (t >> 3);
+  for (int first = 0; first < kDim; first += kFitThreads / 8) {
+    const int column = first + (t >> 3);
     const int offset = 16 * (t & 7);
     const uint32_t* src = reinterpret_cast<const uint32_t*>(&sh.code[column * kCodeStride + offset]);
     *reinterpret_cast<uint4*>(a.next_residual + state * kTile + column * kDim + offset) =
@@ -475,11 +647,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
   }
 
   // ---- new compensators, cleared window, position ----------------------------
-  for (int i = t; i < kDim * kRank; i += kThreads) {
+  for (int i = t; i < kDim * kRank; i += kFitThreads) {
     a.next_comp_keys[vb * kRank + i] = sh.nk[i];
     a.next_comp_values[vb * kRank + i] = sh.nv[i];
   }
-  for (int i = t; i < kWindow * kDim / 2; i += kThreads) {
+  for (int i = t; i < kWindow * kDim / 2; i += kFitThreads) {
     reinterpret_cast<uint32_t*>(a.record_keys + rb * kDim)[i] = 0u;
     reinterpret_cast<uint32_t*>(a.record_corrections + rb * kDim)[i] = 0u;
   }
@@ -562,8 +734,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
   // 64 lanes' word writes in distinct banks), so that only one packed word is
   // live at a time.
   uint32_t quad = 0u;
-  reencode_rows(sh, bs, t, a.workspace + state * kTile, a.next_smoothing + vb, a.next_scales + vb,
-                [&](auto c, int8_t code) {
+  float cell[kDim];
+  reencode_rows<true>(sh, cell, true, bs, t, a.workspace + state * kTile, a.next_smoothing + vb,
+                      a.next_scales + vb, [&](auto c, int8_t code) {
                   constexpr int column = decltype(c)::value;
                   quad |= static_cast<uint32_t>(static_cast<uint8_t>(code)) << (8 * (column % 4));
                   if constexpr (column % 4 == 3) {
@@ -639,10 +812,12 @@ int32_t launch_power_refit(void* stream, const int8_t* residual, const float* sm
                        next_scales, next_comp_keys, next_comp_values, residual_workspace,
                        power_iterations};
   void* pointers[] = {const_cast<PowerArgs*>(&args)};
-  const hipError_t status =
-      hipLaunchKernel(reinterpret_cast<const void*>(power_refit_kernel), dim3(states),
-                      dim3(kThreads), pointers, sizeof(PowerShared),
-                      static_cast<hipStream_t>(stream));
+  const bool split = states <= kSplitStates;
+  const hipError_t status = hipLaunchKernel(
+      split ? reinterpret_cast<const void*>(power_refit_kernel<true>)
+            : reinterpret_cast<const void*>(power_refit_kernel<false>),
+      dim3(states), dim3(split ? kSplitThreads : kThreads), pointers, sizeof(PowerShared),
+      static_cast<hipStream_t>(stream));
   return status == hipSuccess ? kStatusOk : kStatusLaunchFailed;
 }
 

@@ -296,3 +296,50 @@ def test_quant_only_refit_at_fp16_ties(device):
     W.window_boundary_quant_only(ref, ref_out)
     assert_same(from_device(do, out), ref_out, OUT_NAMES)
     assert_same(from_device(d, buf), ref, buf.keys())
+
+
+def test_power_refit_forms_agree_at_their_line(device):
+    """768 states take the split form of the power refit, 769 the whole one:
+    the states they share come out bit for bit the same, among them windows
+    whose first normalization fails (all zero), whose norms lie above 2^32 or
+    below 2^-32 (the root's 20 steps) and whose compensators dominate.  Every
+    128th state and the planted ones against the oracle."""
+    states = 769
+    from test_boundary_oracle import planted_window
+
+    few = planted_window(32, 91)
+    buf = {k: np.ascontiguousarray(np.resize(v, (states,) + v.shape[1:])) for k, v in few.items()}
+    buf["positions"][:, 0] = 16
+    rng = np.random.default_rng(92)
+    buf["record_decay"][:] = 0.9 + 0.1 * rng.random(buf["record_decay"].shape, np.float32)
+    buf["scales"] *= (0.5 + rng.random(buf["scales"].shape, np.float32))
+    for name in ("residual", "record_keys", "record_corrections", "compensator_keys",
+                 "compensator_values"):
+        buf[name][5] = 0
+    buf["scales"][6] *= np.float32(2.0 ** 40)
+    buf["scales"][7] *= np.float32(2.0 ** -40)
+    buf["record_keys"][7] = 0
+    buf["compensator_keys"][7] = 0
+    buf["compensator_keys"][8] = np.float16(30.0).view(np.uint16)
+    print(f"power refit forms, states={states}", flush=True)
+    results = []
+    for count in (states, states - 1):
+        part = {k: v[:count] for k, v in buf.items()}
+        out = sentinel_outputs(count)
+        d, do = to_device(part, device), to_device(out, device)
+        dw = torch.full((count, 128, 128), 7.0, dtype=torch.float32, device=device)
+        assert native().window_boundary_launch_v1(
+            stream(), *window_ptrs(d), *out_ptrs(do), dw.data_ptr(), count, 3) == 0
+        torch.cuda.synchronize()
+        results.append((from_device(do, out), from_device(d, part), dw.cpu().numpy()))
+    (whole, whole_buf, whole_ws), (split, split_buf, split_ws) = results
+    first = np.arange(states - 1)
+    assert_same(_subset(whole, first), split, OUT_NAMES)
+    assert_same(_subset(whole_buf, first), split_buf, buf.keys())
+    assert whole_ws[:-1].tobytes() == split_ws.tobytes()
+    idx = np.unique(np.r_[np.arange(0, 16), np.arange(0, states, 128), states - 1])
+    ref, ref_out = _subset(buf, idx), _subset(sentinel_outputs(states), idx)
+    ref_ws = np.full((idx.size, 128, 128), 7.0, np.float32)
+    W.window_boundary_power(ref, ref_out, ref_ws, 3)
+    assert_same(_subset(whole, idx), ref_out, OUT_NAMES)
+    assert whole_ws[idx].tobytes() == ref_ws.tobytes()
