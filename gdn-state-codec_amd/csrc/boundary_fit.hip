@@ -19,13 +19,19 @@
 // One 128-thread workgroup per head; thread t holds residual row t in 128
 // VGPRs.  Row sums (left = R right, the singular value's products, the update)
 // read the thread's own registers.  Column sums (right = R^T left) need the
-// transpose: the rows are staged through LDS 64 at a time, column-major (a
-// 34 KiB buffer, so four heads fit in a CU's LDS where the whole 66 KiB
-// residual allowed two), and thread t sums column t in row order.  Each norm's terms are the exact
-// double squares of the vector's elements, which their owners publish in LDS
-// beside the vector; every thread then runs the reference's sequential sum over
-// them.  The singular value's 16,384 products are formed by the row owners,
-// staged 64 rows at a time, and summed in the reference's order by one lane.
+// transpose, which changes only with the rank: at its start the rows are staged
+// through LDS 64 at a time, column-major, and thread t keeps rows 64..127 of
+// column t in 64 more VGPRs while rows 0..63 stay in the 34 KiB buffer (four
+// heads then share a CU's LDS and its registers, where a whole transpose in
+// either would allow two).  Each norm's terms are the exact double squares of
+// the vector's elements, which their owners publish in LDS beside the vector;
+// every thread then runs the reference's sequential sum over them.  The singular
+// value's 16,384 products are formed by the row owners, staged 64 rows at a
+// time, and summed in the reference's order by one lane.
+//
+// What bounds it are the dependent sums: 512 terms an iteration, 128 iterations,
+// and 4 x 16,384 terms.  960 heads, rank 4, with the quant stage: 1,243 us with
+// the rows staged through LDS in every iteration, 940 us so.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -143,6 +149,19 @@ __device__ __forceinline__ float relay(const float* chunk, float total) {
   return total;
 }
 
+// Row `line` of the 64 staged rows, column-major, one 4-byte write per value
+// from a single base address (volatile, so none are merged): contiguous writes
+// are merged into 16-byte ones, which need the row in aligned register quads,
+// and paired 4-byte writes need a base address per few columns, which the
+// compiler keeps live.
+__device__ __forceinline__ void stage_rows(FitShared& sh, int line, const float (&row)[kDim]) {
+  typedef __attribute__((address_space(3))) float LdsFloat;
+  volatile LdsFloat* dst = (volatile LdsFloat*)(sh.chunk + line);
+  unrolled<kDim>([&](auto c) {
+    dst[decltype(c)::value * kColumnStride] = row[decltype(c)::value];
+  });
+}
+
 __global__ __launch_bounds__(kFitThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void boundary_fit_kernel(FitArgs a, StartVectors start) {
   extern __shared__ __align__(16) unsigned char dynamic[];
@@ -170,6 +189,17 @@ void boundary_fit_kernel(FitArgs a, StartVectors start) {
   }
 
   for (uint32_t rank = 0; rank < a.rank; ++rank) {
+    // The transpose of the rank's residual: rows 64..127 through the staging
+    // buffer into registers, then rows 0..63, which stay in it.
+    float lower[kChunkRows];
+    const float* const column = sh.chunk + t * kColumnStride;
+    if (t >= kChunkRows) stage_rows(sh, t - kChunkRows, row);
+    __syncthreads();
+    unrolled<kChunkRows>([&](auto i) { lower[decltype(i)::value] = column[decltype(i)::value]; });
+    __syncthreads();
+    if (t < kChunkRows) stage_rows(sh, t, row);
+    // The start vector's barriers below publish the staged rows.
+
     float my_left = 0.0f;
     float my_right;
     publish_square(sh, t, start.value[rank][t]);
@@ -197,43 +227,35 @@ void boundary_fit_kernel(FitArgs a, StartVectors start) {
         __syncthreads();
         if (!left_ok) break;  // uniform: every thread formed the same norm
       }
-      {  // right[col] = sum over rows of R[row][col] * left[row] (thread = column),
-         // the rows staged through LDS 64 at a time
+      {  // right[col] = sum over rows of R[row][col] * left[row] (thread = column):
+         // rows 0..63 of the column from LDS, rows 64..127 from registers
         float acc = 0.0f;
-        unrolled<kDim / kChunkRows>([&](auto h) {
-          constexpr int first = decltype(h)::value * kChunkRows;
-          if (h > 0) __syncthreads();  // every thread done with the previous rows
-          if (t / kChunkRows == decltype(h)::value) {
-            // Column-major, one 4-byte write per value from a single base
-            // address (volatile, so none are merged): contiguous writes are
-            // merged into 16-byte ones, which need the row in aligned register
-            // quads, and paired 4-byte writes need a base address per few
-            // columns, which the compiler keeps live through the whole loop.
-            typedef __attribute__((address_space(3))) float LdsFloat;
-            volatile LdsFloat* dst =
-                (volatile LdsFloat*)(sh.chunk + t % kChunkRows);
-            unrolled<kDim>([&](auto c) {
-              dst[decltype(c)::value * kColumnStride] = row[decltype(c)::value];
-            });
-          }
-          __syncthreads();
-          struct Pair8 {
-            float r[8];
-            float l[8];
-          };
-          const float* column = sh.chunk + t * kColumnStride;
-          pipelined<kChunkRows / 8, Pair8>(
-              [&](auto g, Pair8& p) {
-                unrolled<8>([&](auto i) {
-                  constexpr int r = 8 * decltype(g)::value + decltype(i)::value;
-                  p.r[i] = column[r];
-                  p.l[i] = sh.left[first + r];
-                });
-              },
-              [&](auto, const Pair8& p) {
-                unrolled<8>([&](auto i) { acc += p.r[i] * p.l[i]; });
+        struct Pair8 {
+          float r[8];
+          float l[8];
+        };
+        pipelined<kChunkRows / 8, Pair8>(
+            [&](auto g, Pair8& p) {
+              unrolled<8>([&](auto i) {
+                constexpr int r = 8 * decltype(g)::value + decltype(i)::value;
+                p.r[i] = column[r];
+                p.l[i] = sh.left[r];
               });
-        });
+            },
+            [&](auto, const Pair8& p) {
+              unrolled<8>([&](auto i) { acc += p.r[i] * p.l[i]; });
+            });
+        pipelined<kChunkRows / 16, Float16>(
+            [&](auto g, Float16& l) {
+              unrolled<16>([&](auto i) {
+                l.v[i] = sh.left[kChunkRows + 16 * decltype(g)::value + decltype(i)::value];
+              });
+            },
+            [&](auto g, const Float16& l) {
+              unrolled<16>([&](auto i) {
+                acc += lower[16 * decltype(g)::value + decltype(i)::value] * l.v[i];
+              });
+            });
         publish_square(sh, t, acc);
         __syncthreads();
         const bool right_ok = normalize_into(sh, sh.right, t, acc, &my_right);
