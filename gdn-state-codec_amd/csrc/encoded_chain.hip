@@ -11,23 +11,32 @@
 //
 // Here one 256-thread workgroup owns one state for the whole chain.  The
 // state's int8 boundary is read from HBM once, into registers in both
-// orientations (thread t holds 64 codes of row t/2 and 64 codes of column
-// t/2); the bases, records, scales and the vector live in LDS; and each stage
-// is the reference's arithmetic in the reference's order, so every output is
-// bit-identical to the launch-per-stage chain (the stages are restated from
+// orientations: threads 0..127 hold row t, threads 128..255 column t - 128 (32
+// words each); the bases, records, scales and the vector live in LDS; and each
+// stage is the reference's arithmetic in the reference's order, so every output
+// is bit-identical to the launch-per-stage chain (the stages are restated from
 // the kernels in decode_pair.hip and encoded_rank.hip):
 //   prepare : x = fp16(v) * axis, scale = max|x| > 1e-20 ? max|x| / 127 : 1,
 //             q = round(x / scale) (add +-0.5, clamp to +-127, truncate);
 //   product : p = A q or A^T q, exact in int32 (v_dot4_i32_i8);
 //   finish  : the 24 coefficient sums (old ranks, fitted ranks, records) as
 //             sequential fp32 sums, the rows' value with the window's gates,
-//             the sequential squared norm, its 20-step Newton square root and
-//             the fp16 output v / |v|;
+//             the sequential squared norm, its Newton square root and the fp16
+//             output v / |v|;
 //   commit  : the rows' value written as the rank's left basis (fp16) and as
 //             the corrected vector (fp32), the vector as its right basis.
-// The sequential stages (prepare, finish, commit) run in one wavefront, and
-// the role moves to the next wavefront at every stage so that the four SIMDs
-// of a CU share them; the product uses all four.
+//
+// A step is bound by its serial chain and, with eight states per CU, by the
+// VALU issue of the stages that use one wavefront, so the four wavefronts take
+// different parts of it:
+//   1. one wavefront prepares q while another forms the coefficients (both
+//      need only the vector);
+//   2. the pair of wavefronts whose lines the product runs over forms it and
+//      the rows' values, one line per thread, and their squares;
+//   3. one wavefront sums the norm and writes the next vector.
+// Parts 1 and 3 run on the pair that part 2 leaves free.  2,048 states, 8
+// iterations, the chain with its requantize: 529 us with one wavefront
+// per sequential stage and the lines split over thread pairs, 418 us so.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -35,14 +44,13 @@
 #include "gdn_state_codec_window.h"
 #include "lane_exchange.h"
 #include "launch.h"
+#include "pipelined_sum.h"
 #include "window_common.h"
 
 namespace gdn {
 namespace {
 
 constexpr int kChainThreads = 256;
-constexpr int kChainWaves = kChainThreads / 64;
-constexpr int kChainLanes = 64;
 constexpr int kCoefficientRows = 2 * kRank + kWindow;  // old, fitted, records
 constexpr uint32_t kMaxChainIterations = 64;
 
@@ -66,23 +74,26 @@ struct ChainArgs {
 // axis.  A finish with transpose T takes its input on side T and writes on
 // side 1 - T; the forward product (T = 0) maps a right-side vector to the
 // left side.
-// Basis rows are padded to 132 fp16 (66 words): the 24 coefficient lanes,
-// each reading 8 bytes of its own row, then start on banks 2c and hit 48
-// distinct banks; unpadded 256-byte rows put all 24 on one bank.
-constexpr int kBasisStride = kDim + 4;
+// Basis rows are padded to 136 fp16 (68 words): the 24 coefficient lanes, each
+// reading 16 bytes of its own row, then start on banks 4c; unpadded 256-byte
+// rows put all 24 on one bank.
+constexpr int kBasisStride = kDim + 8;
 
 struct ChainShared {
   // basis[side][row][dim], fp16: rows 0..3 the old compensators of that side
   // (transposed from [dim][rank]), 4..7 the fitted ranks, 8..23 the records.
-  uint16_t basis[2][kCoefficientRows][kBasisStride];
+  __attribute__((aligned(16))) uint16_t basis[2][kCoefficientRows][kBasisStride];
   float axis[2][kDim];
-  float decay[kWindow];
+  float suffix[kCoefficientRows];  // of each record's coefficient; 1 for the ranks
+  float boundary_suffix;           // the whole window's decay product
   __attribute__((aligned(16))) uint16_t vector[kDim];  // the current vector, fp16 bits
   __attribute__((aligned(16))) uint32_t q[kDim / 4];  // the quantized vector
-  int32_t p[kDim];        // the projection
-  __attribute__((aligned(16))) float values[kDim];  // the rows' values, for the norm
+  __attribute__((aligned(16))) float values[kDim];   // the rows' values
+  __attribute__((aligned(16))) float squares[kDim];  // and their squares, for the norm
+  __attribute__((aligned(16))) float coefficients[kCoefficientRows];
   float dynamic_scale;
 };
+static_assert(workgroups_by_lds(sizeof(ChainShared)) >= 8, "eight states per CU");
 
 // Vector quantizer rounding of the reference: add +-0.5, clamp, truncate.
 __device__ __forceinline__ int chain_round(float value) {
@@ -112,121 +123,107 @@ __device__ void chain_prepare(ChainShared& sh, int side, int lane) {
   if (lane == 0) sh.dynamic_scale = scale;
 }
 
-// The rows' value of finish_encoded_projection / commit_encoded_rank
-// (encoded_rank.hip encoded_rows_kernel) for a vector on side `in_side`,
-// `ranks` fitted ranks; one wavefront, rows lane and lane + 64.  Returns the
-// two rows' values.
-__device__ void chain_rows(ChainShared& sh, int in_side, uint32_t ranks, int lane,
-                           float (&row_value)[2]) {
-  const int out_side = 1 - in_side;
-  // The sequential coefficient sums, one per lane 0..23, over the vector.
-  // Each term is an fp16 basis value times an fp16 vector value, a product
-  // exact in fp32, so `coefficient += b * x` rounds exactly what
-  // fma(b, x, coefficient) rounds: one v_fma_mix_f32 per term, reading both
-  // halves of the packed words itself.
+// The coefficients of a vector on side `in_side`, one per lane 0..23 of one
+// wavefront: sequential sums over the vector, the records' times their suffix.
+// Each term is an fp16 basis value times an fp16 vector value, a product exact
+// in fp32, so `coefficient += b * x` rounds exactly what
+// fma(b, x, coefficient) rounds: one v_fma_mix_f32 per term, reading both
+// halves of the packed words itself.
+__device__ void chain_coefficients(ChainShared& sh, int in_side, int lane) {
+  if (lane >= kCoefficientRows) return;
+  const uint16_t* const basis = sh.basis[in_side][lane];
+  const auto term = [](uint32_t b, uint32_t x, float total) {
+    return __builtin_fmaf(half_bits_to_float(b), half_bits_to_float(x), total);
+  };
+  struct Terms8 {
+    uint4 b, x;
+  };
   float coefficient = 0.0f;
-  if (lane < kCoefficientRows) {
-    const uint16_t* const basis = sh.basis[in_side][lane];
-    const auto term = [](uint32_t b, uint32_t x, float total) {
-      return __builtin_fmaf(half_bits_to_float(b), half_bits_to_float(x), total);
-    };
-    for (int i = 0; i < kDim; i += 4) {
-      const uint2 b = *reinterpret_cast<const uint2*>(basis + i);
-      const uint2 x = *reinterpret_cast<const uint2*>(sh.vector + i);
-      coefficient = term(b.x, x.x, coefficient);
-      coefficient = term(b.x >> 16, x.x >> 16, coefficient);
-      coefficient = term(b.y, x.y, coefficient);
-      coefficient = term(b.y >> 16, x.y >> 16, coefficient);
-    }
-  }
-  // Record coefficients times their suffixes, and the whole window's product.
-  float suffix = 1.0f;
-  for (int j = kWindow - 1; j >= 0; --j) {
-    if (lane == 2 * kRank + j) coefficient *= suffix;
-    suffix *= sh.decay[j];
-  }
-  const float boundary_suffix = suffix;
-  float old_coefficient[kRank], new_coefficient[kRank], record_coefficient[kWindow];
+  pipelined<kDim / 8, Terms8>(
+      [&](auto g, Terms8& r) {
+        r.b = *reinterpret_cast<const uint4*>(basis + 8 * decltype(g)::value);
+        r.x = *reinterpret_cast<const uint4*>(sh.vector + 8 * decltype(g)::value);
+      },
+      [&](auto, const Terms8& r) {
+        coefficient = term(r.b.x, r.x.x, coefficient);
+        coefficient = term(r.b.x >> 16, r.x.x >> 16, coefficient);
+        coefficient = term(r.b.y, r.x.y, coefficient);
+        coefficient = term(r.b.y >> 16, r.x.y >> 16, coefficient);
+        coefficient = term(r.b.z, r.x.z, coefficient);
+        coefficient = term(r.b.z >> 16, r.x.z >> 16, coefficient);
+        coefficient = term(r.b.w, r.x.w, coefficient);
+        coefficient = term(r.b.w >> 16, r.x.w >> 16, coefficient);
+      });
+  sh.coefficients[lane] = coefficient * sh.suffix[lane];
+}
+
+// The row's value of finish_encoded_projection / commit_encoded_rank
+// (encoded_rank.hip encoded_rows_kernel) from its projection p, on the output
+// side, with `ranks` fitted ranks.  A basis value times a coefficient is
+// fma(b, c, -0): the rounded product of the widened half in one v_fma_mix_f32.
+__device__ __forceinline__ float chain_row(const ChainShared& sh, int out_side, uint32_t ranks,
+                                           int row, int p, float neg_zero) {
+  float c[kCoefficientRows];
+  unrolled<2 * kRank / 4>([&](auto g) {
+    const float4 v = *reinterpret_cast<const float4*>(sh.coefficients + 4 * decltype(g)::value);
+    c[4 * g] = v.x, c[4 * g + 1] = v.y, c[4 * g + 2] = v.z, c[4 * g + 3] = v.w;
+  });
+  const auto product = [&](int r, float coefficient) {
+    return __builtin_fmaf(half_bits_to_float(sh.basis[out_side][r][row]), coefficient, neg_zero);
+  };
+  const float boundary_suffix = sh.boundary_suffix;
+  float value = static_cast<float>(p) * sh.dynamic_scale / 127.0f * sh.axis[out_side][row] *
+                boundary_suffix;
 #pragma unroll
   for (int r = 0; r < kRank; ++r) {
-    old_coefficient[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(coefficient), r));
-    new_coefficient[r] =
-        __int_as_float(__builtin_amdgcn_readlane(__float_as_int(coefficient), kRank + r));
+    value += product(r, c[r]) * boundary_suffix;
+    const float fitted = product(kRank + r, c[kRank + r]);
+    value -= static_cast<uint32_t>(r) < ranks ? fitted : 0.0f;  // x - 0 is x for every x
   }
 #pragma unroll
-  for (int j = 0; j < kWindow; ++j) {
-    record_coefficient[j] =
-        __int_as_float(__builtin_amdgcn_readlane(__float_as_int(coefficient), 2 * kRank + j));
+  for (int j = 0; j < kWindow; j += 4) {
+    const float4 v = *reinterpret_cast<const float4*>(sh.coefficients + 2 * kRank + j);
+    value += product(2 * kRank + j, v.x);
+    value += product(2 * kRank + j + 1, v.y);
+    value += product(2 * kRank + j + 2, v.z);
+    value += product(2 * kRank + j + 3, v.w);
   }
-  const float dynamic = sh.dynamic_scale;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int row = lane + h * kChainLanes;
-    float value = static_cast<float>(sh.p[row]) * dynamic / 127.0f * sh.axis[out_side][row] *
-                  boundary_suffix;
-#pragma unroll
-    for (int r = 0; r < kRank; ++r) {
-      value += half_bits_to_float(sh.basis[out_side][r][row]) * old_coefficient[r] *
-               boundary_suffix;
-      if (static_cast<uint32_t>(r) < ranks) {
-        value -= half_bits_to_float(sh.basis[out_side][kRank + r][row]) * new_coefficient[r];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kWindow; ++j) {
-      value += half_bits_to_float(sh.basis[out_side][2 * kRank + j][row]) * record_coefficient[j];
-    }
-    row_value[h] = value;
-  }
+  return value;
 }
 
-// finish_encoded_projection: the new vector v / |v| in fp16.
-__device__ void chain_finish(ChainShared& sh, int in_side, uint32_t ranks, int lane) {
-  float row_value[2];
-  chain_rows(sh, in_side, ranks, lane, row_value);
-  sh.values[lane] = row_value[0];
-  sh.values[lane + kChainLanes] = row_value[1];
-  wave_lds_sync();
+// The end of finish_encoded_projection: the new vector v / |v| in fp16, by one
+// wavefront, rows 2l, 2l + 1.
+__device__ void chain_normalize(ChainShared& sh, int lane) {
+  struct Squares8 {
+    float4 a, b;
+  };
   float squared_norm = 0.0f;
-  for (int row = 0; row < kDim; row += 4) {
-    const float4 v = *reinterpret_cast<const float4*>(sh.values + row);
-    squared_norm += v.x * v.x;
-    squared_norm += v.y * v.y;
-    squared_norm += v.z * v.z;
-    squared_norm += v.w * v.w;
-  }
+  pipelined<kDim / 8, Squares8>(
+      [&](auto g, Squares8& r) {
+        r.a = *reinterpret_cast<const float4*>(sh.squares + 8 * decltype(g)::value);
+        r.b = *reinterpret_cast<const float4*>(sh.squares + 8 * decltype(g)::value + 4);
+      },
+      [&](auto, const Squares8& r) {
+        squared_norm += r.a.x;
+        squared_norm += r.a.y;
+        squared_norm += r.a.z;
+        squared_norm += r.a.w;
+        squared_norm += r.b.x;
+        squared_norm += r.b.y;
+        squared_norm += r.b.z;
+        squared_norm += r.b.w;
+      });
   const float inverse = squared_norm > 1.0e-20f ? 1.0f / newton_sqrt(squared_norm) : 0.0f;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int row = lane + h * kChainLanes;
-    sh.vector[row] = static_cast<uint16_t>(float_to_half_bits(row_value[h] * inverse));
-  }
+  const float2 v = *reinterpret_cast<const float2*>(sh.values + 2 * lane);
+  reinterpret_cast<uint32_t*>(sh.vector)[lane] =
+      (float_to_half_bits(v.x * inverse) & 0xFFFFu) | (float_to_half_bits(v.y * inverse) << 16);
 }
 
-// commit_encoded_rank of rank `rank` (its vector on the right side).
-__device__ void chain_commit(ChainShared& sh, const ChainArgs& a, uint64_t state, uint32_t rank,
-                             int lane) {
-  float row_value[2];
-  chain_rows(sh, 0, rank, lane, row_value);
-  const uint64_t base = (state * kRank + rank) * kDim;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int row = lane + h * kChainLanes;
-    const uint16_t left = static_cast<uint16_t>(float_to_half_bits(row_value[h]));
-    const uint16_t right = sh.vector[row];
-    a.corrected[base + row] = row_value[h];
-    a.new_left[base + row] = left;
-    a.new_right[base + row] = right;
-    sh.basis[1][kRank + rank][row] = left;
-    sh.basis[0][kRank + rank][row] = right;
-  }
-}
-
-// sum over i < 16 of the signed byte dot products of codes[i] and q[i].
-__device__ __forceinline__ int dot64(const uint32_t (&codes)[16], const uint32_t* q) {
+// Signed byte dot product of the thread's line and q, exact in int32.
+__device__ __forceinline__ int chain_dot(const uint32_t (&codes)[kDim / 4], const uint32_t* q) {
   int acc = 0;
 #pragma unroll
-  for (int i = 0; i < 16; i += 4) {
+  for (int i = 0; i < kDim / 4; i += 4) {
     const uint4 qw = *reinterpret_cast<const uint4*>(q + i);
     acc = __builtin_amdgcn_sdot4(static_cast<int>(codes[i]), static_cast<int>(qw.x), acc, false);
     acc = __builtin_amdgcn_sdot4(static_cast<int>(codes[i + 1]), static_cast<int>(qw.y), acc,
@@ -240,61 +237,54 @@ __device__ __forceinline__ int dot64(const uint32_t (&codes)[16], const uint32_t
 }
 
 // Eight waves per SIMD (64 VGPRs): two states per SIMD at a time and 2,048 in
-// flight, so 8,192 states run in four full rounds.  The compiler spills about
-// half of the column words to scratch and reloads them in each transposed
-// product; measured at 8,192 states and 8 iterations (ms): 2.20 at five waves
-// per SIMD without spills, 1.99 at six, 1.76 at eight, bit-identical.
+// flight, so 8,192 states run in four full rounds.
 __global__ __launch_bounds__(kChainThreads, 8) void encoded_chain_kernel(ChainArgs a) {
   __shared__ ChainShared sh;
   const int t = threadIdx.x;
   const int wave = t >> 6;
   const int lane = t & 63;
+  const int pair = t >> 7;            // 0: the rows' wavefronts, 1: the columns'
+  const int line = t & (kDim - 1);
   const uint64_t state = blockIdx.x;
 
   // ---- the boundary in registers, both orientations ------------------------
-  // rows[i]: codes A[t/2][64 (t&1) + 4i ..+3]; columns[i]: codes
-  // A[64 (t&1) + 4i + j][t/2], j = 0..3, one word each.
-  const int line = t >> 1;
-  const int part = t & 1;
+  // codes[i]: A[line][4i ..+3] in a row's thread, A[4i ..+3][line] in a
+  // column's, whose bytes come through LDS, half the tile at a time, staged in
+  // the basis area before the bases are loaded.
   const int8_t* const tile = a.residual + state * kTile;
-  uint32_t rows[16], columns[16];
-  {
-    const uint4* src = reinterpret_cast<const uint4*>(tile + line * kDim + 64 * part);
+  uint32_t codes[kDim / 4];
+  if (pair == 0) {
+    const uint4* src = reinterpret_cast<const uint4*>(tile + line * kDim);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kDim / 16; ++i) {
       const uint4 w = src[i];
-      rows[4 * i] = w.x, rows[4 * i + 1] = w.y, rows[4 * i + 2] = w.z, rows[4 * i + 3] = w.w;
+      codes[4 * i] = w.x, codes[4 * i + 1] = w.y, codes[4 * i + 2] = w.z, codes[4 * i + 3] = w.w;
     }
-    // The columns through LDS, half the tile at a time, staged in the basis
-    // area before the bases are loaded: rows 64h..64h+63 (8 KiB) are written
-    // by the threads that hold them and read down the columns by the threads
-    // of part h.
-    uint8_t* const stage = reinterpret_cast<uint8_t*>(&sh.basis[0][0][0]);
-    static_assert(sizeof(sh.basis) >= 64 * kDim, "staging area");
+  }
+  uint8_t* const stage = reinterpret_cast<uint8_t*>(&sh.basis[0][0][0]);
+  static_assert(sizeof(sh.basis) >= kDim / 2 * kDim, "staging area");
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      __syncthreads();
-      if ((line >> 6) == h) {
-        uint4* const to = reinterpret_cast<uint4*>(stage + (line - 64 * h) * kDim + 64 * part);
+  for (int h = 0; h < 2; ++h) {
+    if (wave == h) {
+      uint4* const to = reinterpret_cast<uint4*>(stage + lane * kDim);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          to[i] = make_uint4(rows[4 * i], rows[4 * i + 1], rows[4 * i + 2], rows[4 * i + 3]);
-        }
-      }
-      __syncthreads();
-      if (part == h) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          uint32_t word = 0;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            word |= static_cast<uint32_t>(stage[(4 * i + j) * kDim + line]) << (8 * j);
-          }
-          columns[i] = word;
-        }
+      for (int i = 0; i < kDim / 16; ++i) {
+        to[i] = make_uint4(codes[4 * i], codes[4 * i + 1], codes[4 * i + 2], codes[4 * i + 3]);
       }
     }
-    __syncthreads();  // the staging area becomes the bases
+    __syncthreads();
+    if (pair == 1) {
+#pragma unroll
+      for (int i = 0; i < kDim / 8; ++i) {
+        uint32_t word = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          word |= static_cast<uint32_t>(stage[(4 * i + j) * kDim + line]) << (8 * j);
+        }
+        codes[kDim / 8 * h + i] = word;
+      }
+    }
+    __syncthreads();  // the staging area becomes the second half, then the bases
   }
 
   // ---- bases, records, scales, gates, zero fitted ranks --------------------
@@ -315,39 +305,56 @@ __global__ __launch_bounds__(kChainThreads, 8) void encoded_chain_kernel(ChainAr
   if (t < kDim) {
     sh.axis[0][t] = a.scales[state * kDim + t];
     sh.axis[1][t] = a.smoothing[state * kDim + t];
+    sh.vector[t] = a.seeds[state * kRank * kDim + t];
   }
-  if (t < kWindow) sh.decay[t] = a.record_decay[state * kWindow + t];
+  if (t == kDim) {
+    float suffix = 1.0f;
+    for (int j = kWindow - 1; j >= 0; --j) {
+      sh.suffix[2 * kRank + j] = suffix;
+      suffix *= a.record_decay[state * kWindow + j];
+    }
+    for (int r = 0; r < 2 * kRank; ++r) sh.suffix[r] = 1.0f;
+    sh.boundary_suffix = suffix;
+  }
+  __syncthreads();
 
   // ---- the chain -----------------------------------------------------------
-  int role = 0;  // the wavefront that runs the next sequential stage
+  const float neg_zero = opaque_negative_zero();
   for (uint32_t rank = 0; rank < static_cast<uint32_t>(kRank); ++rank) {
-    __syncthreads();  // the previous rank's commit has read the vector
-    if (t < kDim) sh.vector[t] = a.seeds[(state * kRank + rank) * kDim + t];
     const uint32_t steps = 2 * a.iterations + 1;  // forward, transposed, ..., commit
     for (uint32_t step = 0; step < steps; ++step) {
-      const int side = static_cast<int>(step & 1u);  // input side: 0 forward, 1 transposed
+      // Input side 0 forward, 1 transposed; the product's lines are those of
+      // pair `side`, the other pair's two wavefronts take the parts beside it,
+      // exchanged from one iteration to the next.
+      const int side = static_cast<int>(step & 1u);
+      const int first = 2 * (1 - side) + static_cast<int>((step >> 1) & 1u);
+      const int second = first ^ 1;
+      if (wave == first) chain_prepare(sh, side, lane);
+      if (wave == second) chain_coefficients(sh, side, lane);
       __syncthreads();
-      if (wave == role) chain_prepare(sh, side, lane);
-      __syncthreads();
-      // p[line] over the thread's 64 codes of the line and its partner's 64
-      // (a uniform branch: one straight loop per orientation, no selects).
-      int acc = 0;
-      if (side == 0) {
-        acc = dot64(rows, sh.q + 16 * part);
-      } else {
-        acc = dot64(columns, sh.q + 16 * part);
-      }
-      acc += __builtin_amdgcn_update_dpp(0, acc, 0xB1, 0xF, 0xF, false);  // partner lane t ^ 1
-      if (part == 0) sh.p[line] = acc;
-      __syncthreads();
-      if (wave == role) {
+      if (pair == side) {
+        const int p = chain_dot(codes, sh.q);
+        const float value = chain_row(sh, 1 - side, rank, line, p, neg_zero);
         if (step + 1 < steps) {
-          chain_finish(sh, side, rank, lane);
-        } else {
-          chain_commit(sh, a, state, rank, lane);
+          sh.values[line] = value;
+          sh.squares[line] = value * value;
+        } else {  // commit_encoded_rank, the vector on the right side
+          const uint64_t at = (state * kRank + rank) * kDim + line;
+          const uint16_t left = static_cast<uint16_t>(float_to_half_bits(value));
+          const uint16_t right = sh.vector[line];
+          a.corrected[at] = value;
+          a.new_left[at] = left;
+          a.new_right[at] = right;
+          sh.basis[1][kRank + rank][line] = left;
+          sh.basis[0][kRank + rank][line] = right;
+          if (rank + 1 < static_cast<uint32_t>(kRank)) sh.vector[line] = a.seeds[at + kDim];
         }
       }
-      role = (role + 1) & (kChainWaves - 1);
+      __syncthreads();
+      if (step + 1 < steps) {
+        if (wave == second) chain_normalize(sh, lane);
+        __syncthreads();
+      }
     }
   }
 }
