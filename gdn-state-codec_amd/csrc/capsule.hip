@@ -3,11 +3,11 @@
 // Serialize = capsule_pack_kernel (one 256-thread workgroup per state: header,
 // codes transposed to the capsule's [key][value] order through LDS, fp16 ->
 // fp32 widening of compensators and records; coalesced 4/8-byte stores) then
-// capsule_digest_kernel<false> (one lane per capsule: SHA-256 of the content,
+// capsule_digest_kernel<false> (two lanes per capsule: SHA-256 of the content,
 // written as 64 lowercase hex characters after it).
 //
 // Restore = capsule_digest_kernel<true> (extent, length, magic, digest
-// encoding and digest checks; one lane per capsule) then capsule_unpack_kernel
+// encoding and digest checks; two lanes per capsule) then capsule_unpack_kernel
 // (one workgroup per state: the remaining checks of
 // GdnStateCodecCapsule::Restore in the reference's order -- parameters,
 // identity, window position and phase, codes != -128, boundary payload,
@@ -15,10 +15,10 @@
 // check, and only then the slot writes).
 //
 // SHA-256 is a serial chain per message (FIPS 180-4 section 6.2), so the
-// digest kernel gives each capsule one lane and is bound by integer VALU
-// issue, not HBM: a producer wavefront expands each 64-byte block's message
-// schedule and the consumer's round chain is about 900 VALU instructions per
-// block.  The pack and unpack kernels move 22-45 KB per state and are
+// digest kernel gives each capsule two lanes, one per half of the round, and is
+// bound by integer VALU issue, not HBM: a producer wavefront expands each
+// 64-byte block's message schedule and the consumer's round chain is about 710
+// VALU instructions per block.  The pack and unpack kernels move 22-45 KB per state and are
 // HBM-bound.
 #include <hip/hip_runtime.h>
 #include <float.h>
@@ -26,6 +26,7 @@
 #include <string.h>
 
 #include "gdn_state_codec_capsule.h"
+#include "lane_exchange.h"
 #include "launch.h"
 #include "window_common.h"
 
@@ -55,7 +56,8 @@ static_assert(content_bytes(0) + kDigestChars == 21688, "capsule size");
 static_assert(content_bytes(0) % 64 == 56, "the digest tail spans two blocks");
 
 constexpr int kThreads = 256;
-constexpr int kDigestLanes = 64;                 // capsules per digest workgroup
+constexpr int kDigestCapsules = 32;  // per digest workgroup, two lanes each
+constexpr int kDigestLanes = 2 * kDigestCapsules;
 constexpr int kDigestThreads = 2 * kDigestLanes;  // producer + consumer wavefront
 
 // The expected / written identity, as kernel-argument words.
@@ -101,6 +103,11 @@ __device__ __forceinline__ uint32_t choose(uint32_t x, uint32_t y, uint32_t z) {
 }
 __device__ __forceinline__ uint32_t majority(uint32_t x, uint32_t y, uint32_t z) {
   return __builtin_amdgcn_bitop3_b32(x, y, z, 0xE8);  // (x&y) ^ (x&z) ^ (y&z)
+}
+
+// x where mask is 0, ~(x ^ y) where it is all ones.
+__device__ __forceinline__ uint32_t same_where(uint32_t x, uint32_t y, uint32_t mask) {
+  return __builtin_amdgcn_bitop3_b32(x, y, mask, 0xD2);
 }
 
 // Block `block` of the padded message of content[0, size) (FIPS 180-4
@@ -155,11 +162,11 @@ __device__ __forceinline__ void message_block(const uint8_t* content, uint32_t s
 // Compression blocks of the padded message of `size` bytes.
 __device__ __forceinline__ uint32_t message_blocks(uint32_t size) { return (size + 9 + 63) / 64; }
 
-// 16 words of lowercase hex characters of the digest (the reference's
+// 8 words of lowercase hex characters of half a digest (the reference's
 // Sha256Hex string, 4 characters per little-endian word).
-__device__ __forceinline__ void digest_hex(const uint32_t (&h)[8], uint32_t (&hex)[16]) {
+__device__ __forceinline__ void digest_hex(const uint32_t (&h)[4], uint32_t (&hex)[8]) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < 4; ++i) {
     uint32_t chars[2] = {0, 0};
 #pragma unroll
     for (int n = 0; n < 8; ++n) {
@@ -181,27 +188,40 @@ struct DigestArgs {
   uint32_t states;
 };
 
-// One workgroup hashes 64 capsules, one per lane, with two wavefronts: the
+// One workgroup hashes 32 capsules, two lanes each, with two wavefronts: the
 // producer loads each 64-byte block, expands the message schedule and writes
 // K[t] + W[t] for the block's 64 rounds to a double-buffered LDS ring; the
-// consumer runs only the round function from the ring (section 6.2.2), so
-// the serial chain of each capsule carries about two thirds of the
-// instructions of a full compression.  One barrier per block: the producer
-// fills slot b + 1 while the consumer works on slot b, and a slot is
-// refilled only after the barrier the consumer reaches when done with it.
+// consumer runs only the round function from the ring (section 6.2.2).  One
+// barrier per block: the producer fills slot b + 1 while the consumer works on
+// slot b, and a slot is refilled only after the barrier the consumer reaches
+// when done with it.
+//
+// A batch's time is its longest capsule's chain (699 blocks of 64 rounds), one
+// wavefront's VALU issue, whatever the number of lanes at work.  A round's two
+// halves have one shape, Sigma(x0) + f(x0, x1, x2) + m: of a..d with Sigma0, Maj
+// and m = 0, of e..h with Sigma1, Ch and m = h + K + W.  So the even lane of a
+// pair holds a..d, the odd lane e..h, each with its own rotation counts, and
+// both halves go through the same 11 instructions where one lane needs 14:
+// Maj(a, b, c) is Ch(~(a ^ b), b, c); the new a is the sum of both halves and
+// the new e that of d and the odd half, so each lane adds what its partner
+// offers (d, or the odd half) to its own half.  4,096 capsules, serialize and
+// restore: 2,943 us with a lane per capsule, 2,424 us so.
 //
 // kVerify = false: write the digest of each serialized capsule (lengths[i] = 0
 // marks a state the pack kernel skipped).  kVerify = true: the first checks of
 // Restore (state_capsule.cpp:481-494), status[i] = 0 when they all pass.
 template <bool kVerify>
 __global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestArgs a) {
-  __shared__ __align__(16) uint4 ring[2][16][kDigestLanes];  // [slot][round / 4][lane]
+  // [slot][round / 4][lane]; the even lanes' words stay 0.
+  __shared__ __align__(16) uint4 ring[2][16][kDigestLanes];
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const uint32_t s = blockIdx.x * kDigestLanes + lane;
+  const bool odd = (lane & 1) != 0;
+  const uint32_t s = blockIdx.x * kDigestCapsules + (lane >> 1);
 
-  // Per-capsule checks, evaluated identically by both wavefronts so that
-  // their block counts (and so their barrier counts) agree.
+  // Per-capsule checks, evaluated identically by both lanes of a capsule and
+  // both wavefronts so that their block counts (and so their barrier counts)
+  // agree.
   uint32_t status = GDN_STATE_CODEC_CAPSULE_OK;
   bool hash = false;
   uint8_t* base = nullptr;
@@ -259,15 +279,19 @@ __global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestAr
     // ---- producer: message schedule plus round constants ----
     const uint32_t full = content / 64;
     const uint64_t* src = reinterpret_cast<const uint64_t*>(base);
+    if (!odd) {
+#pragma unroll
+      for (int i = 0; i < 32; ++i) ring[i >> 4][i & 15][lane] = make_uint4(0, 0, 0, 0);
+    }
     uint64_t next[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) next[i] = 0;
-    if (full > 0) {
+    if (odd && full > 0) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) next[i] = src[i];
     }
     for (uint32_t block = 0; block < wave_blocks; ++block) {
-      if (block < blocks) {
+      if (odd && block < blocks) {
         uint32_t w[16];
         message_block(base, content, block, next, w);
         // Issue the next block's loads before this block's schedule.
@@ -301,62 +325,75 @@ __global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestAr
     return;
   }
 
-  // ---- consumer: the round chain ----
-  uint32_t h[8];
+  // ---- consumer: the round chain, a..d in the even lane, e..h in the odd ----
+  uint32_t h[4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) h[i] = kInitial[i];
+  for (int i = 0; i < 4; ++i) h[i] = odd ? kInitial[4 + i] : kInitial[i];
+  const uint32_t r0 = odd ? 6 : 2, r1 = odd ? 11 : 13, r2 = odd ? 25 : 22;
+  const uint32_t odd_mask = odd ? ~0u : 0u;
+  const uint32_t even_mask = ~odd_mask;
   for (uint32_t block = 0; block < wave_blocks; ++block) {
     __syncthreads();  // slot (block & 1) is ready
     if (block < blocks) {
       const uint4* slot = &ring[block & 1][0][0];
-      uint32_t va = h[0], vb = h[1], vc = h[2], vd = h[3], ve = h[4], vf = h[5], vg = h[6],
-               vh = h[7];
+      uint32_t x0 = h[0], x1 = h[1], x2 = h[2], x3 = h[3];
+      uint4 kw = slot[lane];
+      uint32_t m = (x3 & odd_mask) + kw.x;
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
-        const uint4 kw4 = slot[q * kDigestLanes + lane];
-        const uint32_t kw[4] = {kw4.x, kw4.y, kw4.z, kw4.w};
+        const uint4 following = slot[(q < 15 ? q + 1 : q) * kDigestLanes + lane];
+        const uint32_t next[4] = {kw.y, kw.z, kw.w, following.x};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const uint32_t t1 = vh + xor3(rotr(ve, 6), rotr(ve, 11), rotr(ve, 25)) +
-                              choose(ve, vf, vg) + kw[i];
-          const uint32_t t2 = xor3(rotr(va, 2), rotr(va, 13), rotr(va, 22)) + majority(va, vb, vc);
-          vh = vg;
-          vg = vf;
-          vf = ve;
-          ve = vd + t1;
-          vd = vc;
-          vc = vb;
-          vb = va;
-          va = t1 + t2;
+          const uint32_t half = xor3(rotr(x0, r0), rotr(x0, r1), rotr(x0, r2)) +
+                                choose(same_where(x0, x1, even_mask), x1, x2) + m;
+          const uint32_t offer = odd ? half : x3;
+          // The next round's m stands between the offer and its cross-lane
+          // read, which must wait two instructions for it; opaque, so that its
+          // terms are not added into the chain instead.
+          __builtin_amdgcn_sched_barrier(0);
+          m = (x2 & odd_mask) + next[i];
+          asm("" : "+v"(m));
+          __builtin_amdgcn_sched_barrier(0);
+          x3 = x2;
+          x2 = x1;
+          x1 = x0;
+          x0 = half + static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(
+                          static_cast<int>(offer), kDppQuadSwap1, 0xF, 0xF, true));
         }
+        kw = following;
       }
-      h[0] += va;
-      h[1] += vb;
-      h[2] += vc;
-      h[3] += vd;
-      h[4] += ve;
-      h[5] += vf;
-      h[6] += vg;
-      h[7] += vh;
+      h[0] += x0;
+      h[1] += x1;
+      h[2] += x2;
+      h[3] += x3;
     }
   }
   if (s >= a.states) return;
   if (!hash) {
-    if constexpr (kVerify) a.status[s] = status;
+    if constexpr (kVerify) {
+      if (!odd) a.status[s] = status;
+    }
     return;
   }
-  uint32_t hex[16];
+  uint32_t hex[8];  // the lane's half of the digest
   digest_hex(h, hex);
   if constexpr (kVerify) {
-    bool same = true;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) same = same && recorded[i] == hex[i];
-    a.status[s] = same ? GDN_STATE_CODEC_CAPSULE_OK : GDN_STATE_CODEC_CAPSULE_DIGEST_MISMATCH;
-  } else {
-    // Serialized content is a multiple of 8 bytes long.
-    uint64_t* out = reinterpret_cast<uint64_t*>(base + content);
+    int same = 1;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
+      same &= static_cast<int>((odd ? recorded[8 + i] : recorded[i]) == hex[i]);
+    }
+    // Both lanes of a pair are here: they evaluated the same checks.
+    same &= __builtin_amdgcn_mov_dpp(same, kDppQuadSwap1, 0xF, 0xF, true);
+    if (!odd) {
+      a.status[s] = same ? GDN_STATE_CODEC_CAPSULE_OK : GDN_STATE_CODEC_CAPSULE_DIGEST_MISMATCH;
+    }
+  } else {
+    // Serialized content is a multiple of 8 bytes long.
+    uint64_t* out = reinterpret_cast<uint64_t*>(base + content) + (odd ? 4 : 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
       out[i] = static_cast<uint64_t>(hex[2 * i]) | (static_cast<uint64_t>(hex[2 * i + 1]) << 32);
     }
   }
@@ -857,7 +894,9 @@ bool make_identity(const char* geometry, uint64_t generation, uint64_t epoch, Id
   return true;
 }
 
-uint32_t digest_blocks(uint32_t states) { return (states + kDigestLanes - 1) / kDigestLanes; }
+uint32_t digest_blocks(uint32_t states) { 
+  return (states + kDigestCapsules - 1) / kDigestCapsules;
+}
 
 }  // namespace
 }  // namespace gdn

@@ -91,6 +91,42 @@ def test_serialize_is_byte_identical_to_the_oracle(device, layout):
         assert np.array_equal(after[name], buf[name]), name
 
 
+@pytest.mark.parametrize("states", [1, 31, 32, 33, 65])
+def test_digests_at_the_edges_of_a_workgroup(device, states):
+    """A digest workgroup takes 32 capsules, two lanes each: batches around
+    that, capsules of unequal length side by side, some skipped or tampered
+    with; byte-identical, and restore's digest check fails for exactly the
+    tampered ones, whichever half of the digest differs."""
+    positions = [(5 * s) % 16 for s in range(states)]
+    print(f"capsule digests states={states}", flush=True)
+    buf = WG.window_buffers(states, 91, VK, positions=positions)
+    want = [C.slot_serialize(buf, s, VK, IDENTITY) for s in range(states)]
+    sizes = [len(w) for w in want]
+    offsets = np.cumsum([0] + sizes[:-1]).astype(np.uint64)
+    skipped = [s for s in range(states) if s % 7 == 3]
+    given = offsets.copy()
+    given[skipped] += 4  # misaligned: not written
+    capacity = int(sum(sizes))
+    got, lengths = serialize_on_gpu(to_device(buf, device), states, VK, given, capacity, device)
+    for s in range(states):
+        o = int(offsets[s])
+        blob = got[o:o + sizes[s]]
+        if s in skipped:
+            assert lengths[s] == 0 and (blob == FILL).all(), s
+            blob[:] = np.frombuffer(want[s], np.uint8)
+        assert blob.tobytes() == want[s], s
+    expect = np.zeros(states, np.int32)
+    for s in range(states):  # one hex character of the recorded digest, either half
+        if s % 3 == 1:
+            at = int(offsets[s]) + sizes[s] - 64 + (11 * s) % 64
+            got[at] = ord("0") if got[at] != ord("0") else ord("1")
+            expect[s] = C.DIGEST_MISMATCH
+    fresh = to_device(WG.window_buffers(states, 92, VK), device)
+    status = restore_on_gpu(got, offsets, np.array(sizes, np.uint32), positions, fresh, states,
+                            VK, device)
+    assert status.tolist() == expect.tolist()
+
+
 def test_serialize_skips_capsules_that_do_not_fit(device):
     states = 4
     print("capsule serialize extent", flush=True)
