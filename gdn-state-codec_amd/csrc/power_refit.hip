@@ -60,6 +60,14 @@ constexpr float kBoundaryFloor = 1.0e-8f;
 // rounds come out full and it is ahead by 16% and 2%, at 1,280 behind by 7%.
 constexpr uint32_t kSplitStates = 768;
 
+// In the form with codes in registers, the values of a row's first columns are
+// held as well: what three wavefronts per SIMD leave of the registers.  Such a
+// value costs an application three VALU instructions, one formed from its code
+// eight.  8,192 states, 4 iterations, with the
+// window's 16 steps: 2,660 us with none held, 2,555 with 48, 2,606 with 64 and
+// 2,729 with 80, where more values are spilled (11, 19 and 35 VGPRs).
+constexpr int kHeldCells = 48;
+
 // f(std::integral_constant<int, c>) for c = 0 .. kDim - 1, expanded at compile
 // time: a body that indexes a register array by c keeps the array in VGPRs,
 // where a loop the compiler declines to unroll fully would move it to scratch.
@@ -219,11 +227,14 @@ __device__ __forceinline__ float line_sum(const float (&cell)[kDim], const float
 }
 
 // The same sum with the line's codes packed four to a word in place of its
-// values; `own` is the line's factor, `across` the other axis' factors, and
-// `rows` tells which of the two is the smoothing (code / 127 * s * scale).
-template <bool kRows>
-__device__ __forceinline__ float code_sum(const uint32_t (&codes)[kDim / 4], const float* vector,
+// values, but for the first kHeld of them, which are in held[]; `own` is the
+// line's factor, `across` the other axis' factors, and `rows` tells which of
+// the two is the smoothing (code / 127 * s * scale).
+template <bool kRows, int kHeld>
+__device__ __forceinline__ float code_sum(const float (&held)[kDim],
+                                          const uint32_t (&codes)[kDim / 4], const float* vector,
                                           const float* across, float own, float bs) {
+  static_assert(kHeld % 4 == 0, "whole code words");
   float value = 0.0f;
   struct Group {
     float x[4], f[4];
@@ -232,9 +243,17 @@ __device__ __forceinline__ float code_sum(const uint32_t (&codes)[kDim / 4], con
       [&](auto g, Group& r) {
         constexpr int first = 4 * decltype(g)::value;
         *reinterpret_cast<float4*>(r.x) = *reinterpret_cast<const float4*>(vector + first);
-        *reinterpret_cast<float4*>(r.f) = *reinterpret_cast<const float4*>(across + first);
+        if constexpr (first >= kHeld) {
+          *reinterpret_cast<float4*>(r.f) = *reinterpret_cast<const float4*>(across + first);
+        }
       },
       [&](auto g, const Group& r) {
+        if constexpr (4 * decltype(g)::value < kHeld) {
+          unrolled<4>([&](auto i) {
+            value += held[4 * decltype(g)::value + decltype(i)::value] * r.x[i] * bs;
+          });
+          return;
+        }
         // Opaque, so that the widened codes are not formed once for all
         // applications and held (spilled) between them.
         uint32_t word = codes[decltype(g)::value];
@@ -539,6 +558,10 @@ __global__ __launch_bounds__(kSplit ? kSplitThreads : kThreads) __attribute__((a
         column_codes[column / 4] =
             *reinterpret_cast<const uint32_t*>(&sh.code[line * kCodeStride + column]);
       }
+      if constexpr (column < kHeldCells) {
+        cell[column] = code_value_arith(static_cast<int8_t>(code)) * sh.smoothing[line] *
+                       sh.scales[column];
+      }
     });
   } else if (rows) {
     const float s = sh.smoothing[line];
@@ -575,9 +598,9 @@ __global__ __launch_bounds__(kSplit ? kSplitThreads : kThreads) __attribute__((a
       if constexpr (kSplit) {
         value = line_sum(cell, in, bs);
       } else if (forward) {
-        value = code_sum<true>(row_codes, in, sh.scales, sh.smoothing[line], bs);
+        value = code_sum<true, kHeldCells>(cell, row_codes, in, sh.scales, sh.smoothing[line], bs);
       } else {
-        value = code_sum<false>(column_codes, in, sh.smoothing, sh.scales[line], bs);
+        value = code_sum<false, 0>(cell, column_codes, in, sh.smoothing, sh.scales[line], bs);
       }
     }
     __syncthreads();
