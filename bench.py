@@ -1351,8 +1351,8 @@ def bench_capsule(steps: int, warmup: int):
     # chain of the longest capsule (window position 15) whatever the number of
     # capsules: the same serialize on an eighth of the batch (every window
     # position still present) takes nearly as long.  The floor of one chain is
-    # its VALU instructions (905 per 64-byte block on the consumer wavefront
-    # in this build: 6 v_alignbit, 4 v_bitop3 and about 4 adds per round) at
+    # its VALU instructions (710 per 64-byte block on the consumer wavefront
+    # in this build: 11 per round, two lanes a capsule) at
     # one instruction per 4 cycles at the 2.4 GHz peak engine clock.
     small = states // 8
     small_slot = capsule_slot(small, dev)
@@ -1375,7 +1375,7 @@ def bench_capsule(steps: int, warmup: int):
     results["serialize_eighth_batch"] = {"capsules": small,
                                          "us_per_batch": _events_ms([(a, b)])[0] / steps * 1e3}
     results["longest_capsule_sha256_blocks"] = longest
-    results["chain_issue_floor_us"] = longest * 905 * 4 / 2.4e3
+    results["chain_issue_floor_us"] = longest * 710 * 4 / 2.4e3
     results["serialize_frac_of_chain_floor"] = (results["chain_issue_floor_us"]
                                                 / results["serialize"]["us_per_batch"])
     _log(f"capsule serialize of {small} capsules: "
