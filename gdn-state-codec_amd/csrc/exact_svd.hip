@@ -1093,6 +1093,7 @@ __global__ __launch_bounds__(kDirectThreads, 2) void exact_svd_direct_kernel(Svd
       }
 #pragma unroll
       for (int i = 0; i < kDim / 2; ++i) cell[i] = source[i * kDim];
+      __syncthreads();  // every wave has read all four vectors
       sh.pivot[wave][0][lane] = z0;
       sh.pivot[wave][0][64 + lane] = z1;
       __syncthreads();
