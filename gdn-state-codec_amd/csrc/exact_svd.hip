@@ -395,6 +395,7 @@ constexpr double kTinyCoupling = 1e-40;                   // floor of a squared 
 constexpr double kZeroColumn = 1e-200;                    // a squared column norm taken as zero
 constexpr double kSmallestRatio = 0x1p-20;                // lambda_4 / lambda_1
 constexpr double kLargestOverlap = 1e-4;                  // |z_r . z_s| before orthogonalization
+constexpr double kSmallestRemainder = 0.5;                // |q|^2 behind the earlier vectors
 constexpr double kLargestResidual = 1e-12;                // |T z - lambda z|, |T| <= 1
 
 typedef double Double4 __attribute__((ext_vector_type(4)));
@@ -974,8 +975,13 @@ __device__ __forceinline__ void unreflect_block(const DirectShared& sh, double (
 // The vectors q_found .. q_(found + fresh - 1) made orthogonal to the earlier
 // ones (twice, so that the result is at rounding level): the rounding of what
 // an earlier pass left lets them lean on those by about 2^-24, and P^T q would
-// hold that part of the larger triplets.
-__device__ __forceinline__ void clear_earlier(double* q, int found, int fresh, int wave,
+// hold that part of the larger triplets.  A vector most of which lies in the
+// earlier ones' span belongs to rounding noise: what is left of P has no part
+// along that span but noise, so its singular value (and every later one) is at
+// the noise's level, and it and all later vectors become zero.  (Left as it
+// is, normalized back to length one, it would add a triplet of P a second
+// time.)  Returns whether every vector stands; the same in every thread.
+__device__ __forceinline__ bool clear_earlier(double* q, int found, int fresh, int wave,
                                               int lane) {
   double q0[kSvdRank], q1[kSvdRank];
 #pragma unroll
@@ -983,6 +989,7 @@ __device__ __forceinline__ void clear_earlier(double* q, int found, int fresh, i
     q0[r] = q[lane * kSvdRank + r];
     q1[r] = q[(64 + lane) * kSvdRank + r];
   }
+  bool stands = true;
 #pragma unroll
   for (int r = 1; r < kSvdRank; ++r) {
     if (r >= found && r < found + fresh) {  // uniform
@@ -994,9 +1001,11 @@ __device__ __forceinline__ void clear_earlier(double* q, int found, int fresh, i
           q1[r] = fma(-overlap, q1[s], q1[r]);
         }
       }
-      const double inverse = 1.0 / sqrt(wave_sum_f64(fma(q0[r], q0[r], q1[r] * q1[r])));
-      q0[r] *= inverse;
-      q1[r] *= inverse;
+      const double square = wave_sum_f64(fma(q0[r], q0[r], q1[r] * q1[r]));
+      stands = stands && square > kSmallestRemainder;  // false for NaN
+      const double inverse = 1.0 / sqrt(square);
+      q0[r] = stands ? q0[r] * inverse : 0.0;
+      q1[r] = stands ? q1[r] * inverse : 0.0;
     }
   }
   __syncthreads();  // every wave has read q
@@ -1005,6 +1014,7 @@ __device__ __forceinline__ void clear_earlier(double* q, int found, int fresh, i
     q[(64 + lane) * kSvdRank + wave] = wave == 1 ? q1[1] : wave == 2 ? q1[2] : q1[3];
   }
   __syncthreads();
+  return stands;
 }
 
 __global__ __launch_bounds__(kDirectThreads, 2) void exact_svd_direct_kernel(SvdArgs a) {
@@ -1130,7 +1140,9 @@ __global__ __launch_bounds__(kDirectThreads, 2) void exact_svd_direct_kernel(Svd
       q[(64 + lane) * kSvdRank + wave] = own1;
     }
     __syncthreads();
-    if (found > 0 && largest > 0.0f) clear_earlier(q, found, fresh, wave, lane);
+    if (found > 0 && largest > 0.0f && !clear_earlier(q, found, fresh, wave, lane)) {
+      fresh = kSvdRank - found;  // the rest stays zero
+    }
     found += fresh;
 
     // ---- keys P^T q (vectors not found yet are zero) ------------------------

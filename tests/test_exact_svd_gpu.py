@@ -214,6 +214,39 @@ def test_direct_and_jacobi_forms_share_a_batch(device, count):
     assert (apart <= 2 * FIT_TOLERANCE * largest).all()
 
 
+def few_line_heads(seed):
+    """Provider heads ([value][key]) with one to three nonzero value rows or
+    key columns, side by side and scattered, and with equal rows: what is left
+    behind the triplets found is rounding noise inside their own span."""
+    g = np.random.default_rng(seed)
+    heads = []
+    for lines in ([0], [0, 1], [0, 1, 2], [127], [125, 126, 127], [5, 60], [5, 60, 101]):
+        head = np.zeros((128, 128))
+        head[lines] = g.standard_normal((len(lines), 128))
+        heads += [head, head.T, 0.01 * head]
+    for lines in ([3, 90], [3, 90, 100], [40, 41, 42, 43]):  # equal rows
+        head = np.zeros((128, 128))
+        head[lines] = g.standard_normal(128)
+        heads += [head, head.T]
+        other = head.copy()
+        other[7] = g.standard_normal(128)
+        heads += [other, other.T]
+    return np.stack(heads).astype(np.float32)
+
+
+def test_heads_of_few_rows_or_columns(device):
+    """Triplets beyond a head's rank are zero or at rounding level, never the
+    earlier ones once more: the fit, the fp16 pair and the residual against the
+    float64 SVD, everything finite."""
+    provider = few_line_heads(900)
+    dense = np.ascontiguousarray(provider.transpose(0, 2, 1))
+    print(f"exact SVD initializer, few rows, heads={len(dense)}", flush=True)
+    _, got = run(dense)
+    for a in got:
+        assert np.isfinite(a.view(np.float16) if a.dtype == np.uint16 else a).all()
+    check_heads(dense, got, rank_deficient=range(len(dense)))
+
+
 def test_residual_may_overwrite_the_provider_state(device):
     """residual naming the provider buffer itself: each cell is read for the
     last time by the thread that writes it."""
