@@ -44,6 +44,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "gdn_state_codec_kernel.h"
 #include "lane_exchange.h"
 #include "launch.h"
@@ -379,8 +381,9 @@ __global__ __launch_bounds__(kSvdThreads) void exact_svd_jacobi_kernel(SvdArgs a
 // therefore keeps only the triplets with lambda_r > 2^-20 lambda_1 (sigma_r >
 // 2^-10 sigma_1).  A head with fewer than four of them (a state of fewer than
 // four tokens has that rank) takes another pass over what is left of P without
-// the triplets found, rounded to fp32: a relative error of 2^-24 in a part
-// below 2^-10 sigma_1.  A second pass costs as much as the first.  Heads whose
+// the triplets found, which the Gram matrix forms in double from P itself (2^-53
+// of sigma_1 is lost, as in any double form; nothing is kept in fewer bits).  A
+// second pass costs as much as the first.  Heads whose
 // eigenvectors come out far from orthogonal (repeated eigenvalues) or with a
 // residual that is not at rounding level are marked pending for the Jacobi
 // kernel.
@@ -416,9 +419,14 @@ struct DirectShared {
     };
     double pivot[kSvdRank][2][kDim];        // forward and backward pivots, then the vectors
   };
-  double inverse_h[kDim];                   // 2 / u.u (0: no reflection)
-  double d[kDim];                           // diagonal
-  double e[kDim];                           // e_i couples i and i + 1; scaled after the reduction
+  union {
+    struct {
+      double inverse_h[kDim];               // 2 / u.u (0: no reflection)
+      double d[kDim];                       // diagonal
+      double e[kDim];                       // e_i couples i and i + 1; scaled after the reduction
+    };
+    double fit[kSvdRank - 1][kDim];         // P^T q of the triplets found, between passes
+  };
   double lambda[kSvdRank];
   double scaled_minor[kSvdRank][2][kDim / 8];
   float wave_max[kDirectThreads / 64];
@@ -684,9 +692,12 @@ __device__ __forceinline__ int count_below(const DirectShared& sh, double x) {
 // rows 16 (4 half + i / 4) + 4 wave + i % 4, so that register v of half h is
 // slot 4 h + v of reflect_block's layout.  fp32 products are exact in double
 // and neither overflow nor vanish, so P is used unscaled and G scaled: its
-// entries are then at most 128.
-__device__ __forceinline__ void gram_matrix(const DirectShared& sh, double (&m)[8][8], int wave,
-                                            int lane, int exponent) {
+// entries are then at most 128.  With kDeflated the operands are what is left
+// of P without the triplets found, formed in double where they are read
+// (q [row][4] and fit [triplet][key], zero for those not found).
+template <bool kDeflated>
+__device__ __forceinline__ void gram_matrix(const DirectShared& sh, const double* q,
+                                            double (&m)[8][8], int wave, int lane, int exponent) {
   const int c = lane & 15;
   Double4 block[2][8];
 #pragma unroll
@@ -694,26 +705,43 @@ __device__ __forceinline__ void gram_matrix(const DirectShared& sh, double (&m)[
 #pragma unroll
     for (int b = 0; b < 8; ++b) block[h][b] = Double4{0.0, 0.0, 0.0, 0.0};
   }
-  const float* const left = sh.stage + (16 * (c >> 2) + 4 * wave + (c & 3)) * kStageStride +
-                            4 * (lane >> 4);
-  const float* const right = sh.stage + c * kStageStride + 4 * (lane >> 4);
+  const int left = 16 * (c >> 2) + 4 * wave + (c & 3);
+  const int keys = 4 * (lane >> 4);
 #pragma unroll 1
   for (int k = 0; k < kDim; k += 16) {
-    float l[2][4], r[4][4];
+    using Operand = std::conditional_t<kDeflated, double, float>;
+    Operand l[2][4], r[4][4];
+    double fit[kSvdRank - 1][4];
+    if constexpr (kDeflated) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      *reinterpret_cast<float4*>(l[h]) =
-          *reinterpret_cast<const float4*>(left + 64 * h * kStageStride + k);
+      for (int i = 0; i < kSvdRank - 1; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) fit[i][j] = sh.fit[i][k + keys + j];
+      }
     }
+    const auto load = [&](Operand(&to)[4], int row) {
+      float cells[4];
+      *reinterpret_cast<float4*>(cells) =
+          *reinterpret_cast<const float4*>(sh.stage + row * kStageStride + k + keys);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        to[j] = cells[j];
+        if constexpr (kDeflated) {
+#pragma unroll
+          for (int i = 0; i < kSvdRank - 1; ++i) {
+            to[j] = fma(-q[row * kSvdRank + i], fit[i][j], to[j]);
+          }
+        }
+      }
+    };
+#pragma unroll
+    for (int h = 0; h < 2; ++h) load(l[h], left + 64 * h);
     // Four blocks of columns, one key of every lane group at a time:
     // successive products go to different accumulators.
 #pragma unroll
     for (int b0 = 0; b0 < 8; b0 += 4) {
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        *reinterpret_cast<float4*>(r[b]) =
-            *reinterpret_cast<const float4*>(right + 16 * (b0 + b) * kStageStride + k);
-      }
+      for (int b = 0; b < 4; ++b) load(r[b], 16 * (b0 + b) + c);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
 #pragma unroll
@@ -974,8 +1002,8 @@ __device__ __forceinline__ void unreflect_block(const DirectShared& sh, double (
 
 // The vectors q_found .. q_(found + fresh - 1) made orthogonal to the earlier
 // ones (twice, so that the result is at rounding level): the rounding of what
-// an earlier pass left lets them lean on those by about 2^-24, and P^T q would
-// hold that part of the larger triplets.  A vector most of which lies in the
+// an earlier pass left lets them lean on those, and P^T q would hold that part
+// of the larger triplets.  A vector most of which lies in the
 // earlier ones' span belongs to rounding noise: what is left of P has no part
 // along that span but noise, so its singular value (and every later one) is at
 // the noise's level, and it and all later vectors become zero.  (Left as it
@@ -1078,7 +1106,12 @@ __global__ __launch_bounds__(kDirectThreads, 2) void exact_svd_direct_kernel(Svd
       const int c = lane & 15;
       const int row = 4 * wave + (lane >> 4);
       double m[8][8];
-      gram_matrix(sh, m, wave, lane, exponent);
+      if (found == 0) {
+        gram_matrix<false>(sh, q, m, wave, lane, exponent);
+      } else {
+        gram_matrix<true>(sh, q, m, wave, lane, exponent);
+        __syncthreads();  // every wave has read q and fit
+      }
       reflect_block<0>(sh, m, row, c);
       reflect_block<1>(sh, m, row, c);
       reflect_block<2>(sh, m, row, c);
@@ -1162,10 +1195,14 @@ __global__ __launch_bounds__(kDirectThreads, 2) void exact_svd_direct_kernel(Svd
 #pragma unroll
     for (int r = 0; r < kSvdRank; ++r) y[r] = sh.partial[0][key][r] + sh.partial[1][key][r];
 
-    if (found < kSvdRank) {  // uniform: stage what is left and go round again
+    if (found < kSvdRank) {  // uniform: stage P again and go round
       if (wave < found) {
         own0 = q[lane * kSvdRank + wave];
         own1 = q[(64 + lane) * kSvdRank + wave];
+      }
+      if (half == 0) {
+#pragma unroll
+        for (int r = 0; r < kSvdRank - 1; ++r) sh.fit[r][key] = y[r];
       }
       __syncthreads();  // the half sums are read
       largest = 0.0f;
@@ -1176,12 +1213,11 @@ __global__ __launch_bounds__(kDirectThreads, 2) void exact_svd_direct_kernel(Svd
         for (int r = 0; r < kSvdRank - 1; ++r) {
           rest = fma(-vectors[i * kSvdRank + r], y[r], rest);
         }
-        const float kept = static_cast<float>(rest);
-        sh.stage[(64 * half + i) * kStageStride + key] = kept;
-        largest = fmaxf(largest, fabsf(kept));
+        sh.stage[(64 * half + i) * kStageStride + key] = cell[i];
+        largest = fmaxf(largest, fabsf(static_cast<float>(rest)));
         if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);
       }
-      continue;  // the staged cells are published by the next pass's barrier
+      continue;  // the staged cells and fits are published by the next pass's barrier
     }
 
     // ---- fp16 compensators, residual --------------------------------------

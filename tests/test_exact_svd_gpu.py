@@ -214,6 +214,27 @@ def test_direct_and_jacobi_forms_share_a_batch(device, count):
     assert (apart <= 2 * FIT_TOLERANCE * largest).all()
 
 
+def test_a_later_pass_keeps_double(device):
+    """A fourth singular value below 2^-10 of the first, so that a second pass
+    finds it, and a fifth 1e-5 below the fourth: how much of the fifth triplet
+    the fit holds shows what that pass worked with.  Weighted with the two
+    singular vectors, the fp32 roundings of the outputs (about 3e-10 of sigma_1
+    a cell in rms) come to about 3e-10; what is left of the head rounded to
+    fp32 before the pass gives 5e-8 and more."""
+    ratio = 2.0 ** -10.5
+    spectrum = np.concatenate([[1.0, 0.5, 0.25, ratio, ratio * (1 - 1e-5)],
+                               ratio * np.linspace(0.9, 0.01, 123)])
+    dense = np.stack([planted_head(seed, spectrum) for seed in range(910, 914)])
+    print("exact SVD initializer, close singular values behind the limit", flush=True)
+    provider, got = run(dense)
+    assert (got[6] == 0).all()
+    for p, residual in zip(host(provider).astype(np.float64), got[5].astype(np.float64)):
+        u, s, vt = np.linalg.svd(p)
+        fit = p - residual
+        assert abs(u[:, 4] @ fit @ vt[3]) <= 3e-9 * s[0]
+        assert abs(u[:, 3] @ fit @ vt[4]) <= 3e-9 * s[0]
+
+
 def few_line_heads(seed):
     """Provider heads ([value][key]) with one to three nonzero value rows or
     key columns, side by side and scattered, and with equal rows: what is left
