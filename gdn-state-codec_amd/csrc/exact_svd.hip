@@ -8,8 +8,8 @@
 //
 // Two kernels share the work, both in double up to their outputs.  The direct
 // form (Gram matrix, Householder tridiagonal form, the four largest
-// eigenpairs; described at its kernel) serves every head but those with
-// repeated singular values among the four, which it marks and the Jacobi form
+// eigenpairs; described at its kernel) serves every head but those it marks
+// (an eigenpair not at rounding level), which the Jacobi form
 // behind it takes; a caller's own sweep limit means Jacobi throughout.
 //
 // The decomposition is unique only up to the signs of each (u, v) pair and,
@@ -383,10 +383,11 @@ __global__ __launch_bounds__(kSvdThreads) void exact_svd_jacobi_kernel(SvdArgs a
 // four tokens has that rank) takes another pass over what is left of P without
 // the triplets found, which the Gram matrix forms in double from P itself (2^-53
 // of sigma_1 is lost, as in any double form; nothing is kept in fewer bits).  A
-// second pass costs as much as the first.  Heads whose
-// eigenvectors come out far from orthogonal (repeated eigenvalues) or with a
-// residual that is not at rounding level are marked pending for the Jacobi
-// kernel.
+// second pass costs as much as the first.  Where vectors lean on each other
+// (repeated eigenvalues), those up to the first that does are kept and another
+// pass finds the rest: at most four passes, 0.2 ms each for 32 heads, where the
+// Jacobi kernel takes about 2 ms.  A head whose first vector's residual is not
+// at rounding level is marked pending for that kernel.
 constexpr int kDirectThreads = 256;
 constexpr int kStageStride = kDim + 4;                    // floats
 constexpr int kVectorStride = 10;                         // doubles: 16 rows of 8, bank-spread
@@ -925,38 +926,39 @@ __device__ __forceinline__ void twisted_vector(DirectShared& sh, double lambda, 
 }
 
 // The first `fresh` vectors made orthogonal, the same in every wavefront, and
-// vector `wave` left in z0 (element lane) and z1 (64 + lane).  Returns whether
-// the eigenpairs are sound: residuals at rounding level, vectors near
-// orthogonal to begin with.
-__device__ __forceinline__ bool orthogonal_vectors(const DirectShared& sh, int fresh, int wave,
-                                                   int lane, double& z0, double& z1) {
-  bool sound = sh.lambda[0] > 0.0;
-  {
-    double q0[kSvdRank], q1[kSvdRank];
+// vector `wave` left in z0 (element lane) and z1 (64 + lane).  Returns how many
+// of them are sound: residuals at rounding level, vectors near orthogonal to
+// begin with.  (The vectors of equal eigenvalues come out as the same vector,
+// or leaning on each other.)
+__device__ __forceinline__ int orthogonal_vectors(const DirectShared& sh, int fresh, int wave,
+                                                  int lane, double& z0, double& z1) {
+  double q0[kSvdRank], q1[kSvdRank];
 #pragma unroll
-    for (int r = 0; r < kSvdRank; ++r) {
-      q0[r] = sh.pivot[r][0][lane];
-      q1[r] = sh.pivot[r][0][64 + lane];
-      sound = sound && (r >= fresh || sh.pivot[r][1][0] < kLargestResidual);  // false for NaN
-    }
-#pragma unroll
-    for (int r = 1; r < kSvdRank; ++r) {
-      if (r >= fresh) break;
-#pragma unroll
-      for (int s = 0; s < r; ++s) {
-        const double overlap = wave_sum_f64(fma(q0[r], q0[s], q1[r] * q1[s]));
-        sound = sound && fabs(overlap) < kLargestOverlap;
-        q0[r] = fma(-overlap, q0[s], q0[r]);
-        q1[r] = fma(-overlap, q1[s], q1[r]);
-      }
-      const double inverse = 1.0 / sqrt(wave_sum_f64(fma(q0[r], q0[r], q1[r] * q1[r])));
-      q0[r] *= inverse;
-      q1[r] *= inverse;
-    }
-    z0 = wave == 0 ? q0[0] : wave == 1 ? q0[1] : wave == 2 ? q0[2] : q0[3];
-    z1 = wave == 0 ? q1[0] : wave == 1 ? q1[1] : wave == 2 ? q1[2] : q1[3];
+  for (int r = 0; r < kSvdRank; ++r) {
+    q0[r] = sh.pivot[r][0][lane];
+    q1[r] = sh.pivot[r][0][64 + lane];
   }
-  return sound;
+  bool sound = sh.lambda[0] > 0.0 && sh.pivot[0][1][0] < kLargestResidual;  // false for NaN
+  int count = sound ? 1 : 0;
+#pragma unroll
+  for (int r = 1; r < kSvdRank; ++r) {
+    if (r >= fresh) break;
+    sound = sound && sh.pivot[r][1][0] < kLargestResidual;
+#pragma unroll
+    for (int s = 0; s < r; ++s) {
+      const double overlap = wave_sum_f64(fma(q0[r], q0[s], q1[r] * q1[s]));
+      sound = sound && fabs(overlap) < kLargestOverlap;
+      q0[r] = fma(-overlap, q0[s], q0[r]);
+      q1[r] = fma(-overlap, q1[s], q1[r]);
+    }
+    const double inverse = 1.0 / sqrt(wave_sum_f64(fma(q0[r], q0[r], q1[r] * q1[r])));
+    q0[r] *= inverse;
+    q1[r] *= inverse;
+    count += sound ? 1 : 0;
+  }
+  z0 = wave == 0 ? q0[0] : wave == 1 ? q0[1] : wave == 2 ? q0[2] : q0[3];
+  z1 = wave == 0 ? q1[0] : wave == 1 ? q1[1] : wave == 2 ? q1[2] : q1[3];
+  return count;
 }
 
 // Reflections 16 kFirst .. 16 kFirst + 15 undone, in one wavefront for all four
@@ -1130,7 +1132,9 @@ __global__ __launch_bounds__(kDirectThreads, 2) void exact_svd_direct_kernel(Svd
       __syncthreads();
       while (fresh > 1 && !(sh.lambda[fresh - 1] > kSmallestRatio * sh.lambda[0])) --fresh;
       // The same in every wave: formed from the same values by the same steps.
-      if (!orthogonal_vectors(sh, fresh, wave, lane, z0, z1)) {  // uniform
+      fresh = __builtin_amdgcn_readfirstlane(
+          orthogonal_vectors(sh, fresh, wave, lane, z0, z1));
+      if (fresh == 0) {  // uniform
         if (t == 0) a.status[head] = kSvdPending;
         return;
       }

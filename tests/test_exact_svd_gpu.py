@@ -235,6 +235,47 @@ def test_a_later_pass_keeps_double(device):
         assert abs(u[:, 3] @ fit @ vt[4]) <= 3e-9 * s[0]
 
 
+def repeated_heads(seed):
+    """Heads whose leading singular values are exactly equal, which the
+    rounding of a planted spectrum to fp32 does not give: equal blocks on the
+    diagonal, a block times a Hadamard matrix, a scaled permutation, equal
+    unit cells with a smaller rest."""
+    g = np.random.default_rng(seed)
+    sylvester = np.array([[1.0]])
+    while len(sylvester) < 128:
+        sylvester = np.block([[sylvester, sylvester], [sylvester, -sylvester]])
+    heads = [np.kron(np.eye(128 // n), g.standard_normal((n, n))) for n in (64, 43, 32, 16, 4)]
+    heads = [np.pad(h, (0, 128 - len(h))) for h in heads]
+    heads += [np.kron(sylvester[:128 // n, :128 // n], g.standard_normal((n, n))) for n in (64, 32)]
+    heads += [sylvester, 0.25 * np.eye(128)[g.permutation(128)]]
+    cells = np.zeros((128, 128))
+    cells[np.arange(6), np.arange(6)] = 2.0
+    cells[6:, 6:] = 0.01 * g.standard_normal((122, 122))
+    return np.stack(heads + [cells]).astype(np.float32)
+
+
+def test_exactly_repeated_singular_values(device):
+    """Where the fourth singular value is above the fifth the product is
+    unique and checked; where it is not, the fit is a rank-4 part of the head
+    that holds its four largest singular values."""
+    dense = repeated_heads(920)
+    print(f"exact SVD initializer, repeated singular values, heads={len(dense)}", flush=True)
+    provider, got = run(dense)
+    assert (got[6] == 0).all()
+    unique = []
+    for h, p in enumerate(host(provider).astype(np.float64)):
+        s = np.linalg.svd(p, compute_uv=False)
+        if s[3] - s[4] > 1e-3 * s[0]:
+            unique.append(h)
+        fit = p - got[5][h].astype(np.float64)
+        left = np.linalg.svd(p - fit, compute_uv=False)
+        # The best rank-4 approximation, and what it leaves.
+        assert abs(np.linalg.norm(p - fit) - np.linalg.norm(s[4:])) <= 1e-6 * s[0], h
+        assert abs(left[0] - s[4]) <= 1e-6 * s[0], h
+    assert len(unique) >= 2
+    check_heads(dense[unique], [g[unique] for g in got])
+
+
 def few_line_heads(seed):
     """Provider heads ([value][key]) with one to three nonzero value rows or
     key columns, side by side and scattered, and with equal rows: what is left
