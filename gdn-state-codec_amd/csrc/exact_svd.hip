@@ -50,6 +50,7 @@
 #include "lane_exchange.h"
 #include "launch.h"
 #include "window_common.h"
+#include "work_order.h"
 
 namespace gdn {
 namespace {
@@ -329,13 +330,13 @@ __device__ void jacobi_head(SvdShared& sh, const SvdArgs& a, uint64_t head, int 
 
 // The Jacobi form over the batch: every head, or the pending ones, whose marks
 // a workgroup reads 512 at a time (one per thread) before it starts on them.
+// The heads are dealt out by dealt_item: pending ones often recur at a period.
 __global__ __launch_bounds__(kSvdThreads) void exact_svd_jacobi_kernel(SvdArgs a) {
   extern __shared__ __align__(16) unsigned char dynamic[];
   SvdShared& sh = *reinterpret_cast<SvdShared*>(dynamic);
   const int t = threadIdx.x;
-  const uint64_t stride = gridDim.x;
-  for (uint64_t first = blockIdx.x; first < a.heads; first += stride * kSvdThreads) {
-    const uint64_t own = first + t * stride;
+  for (uint64_t turn = 0; turn * gridDim.x < a.heads; turn += kSvdThreads) {
+    const uint64_t own = dealt_item(blockIdx.x, turn + t, gridDim.x);
     const bool wanted = own < a.heads && (!a.pending_only || a.status[own] == kSvdPending);
     const uint64_t mask = __ballot(wanted);
     if ((t & 63) == 0) sh.pending[t >> 6] = mask;
@@ -345,7 +346,7 @@ __global__ __launch_bounds__(kSvdThreads) void exact_svd_jacobi_kernel(SvdArgs a
       while (left != 0) {  // uniform
         const int bit = __builtin_ctzll(left);
         left &= left - 1;
-        jacobi_head(sh, a, first + static_cast<uint64_t>(64 * w + bit) * stride, t);
+        jacobi_head(sh, a, dealt_item(blockIdx.x, turn + 64 * w + bit, gridDim.x), t);
         __syncthreads();  // the next head reuses the rows
       }
     }

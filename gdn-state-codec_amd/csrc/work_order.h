@@ -26,4 +26,17 @@ GDN_ORDER_HD uint64_t xcd_contiguous_item(uint64_t block, uint64_t blocks) {
   return (block & 7u) * per_xcd + (block >> 3);
 }
 
+// Item of turn `turn` of workgroup `block` of `blocks` (at or past the item count
+// where there is none), for items of which few, unknown beforehand, cost any
+// time.  Each turn takes `blocks` items in a row, rotated by kDealStep from the
+// turn before, so that costly items at a period (the same head of every layer)
+// do not all come to the same workgroups.  Over 256 workgroups the fullest one
+// gets at most 3 times its even share of 960 items (the even share being one),
+// 11 times that of 61,440, for every period to 1,024 and its offsets 0, a third
+// and the last; without the rotation 4 and 240 times.
+constexpr uint64_t kDealStep = 101;
+GDN_ORDER_HD uint64_t dealt_item(uint64_t block, uint64_t turn, uint64_t blocks) {
+  return turn * blocks + (block + kDealStep * turn) % blocks;
+}
+
 }  // namespace gdn

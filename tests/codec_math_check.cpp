@@ -44,6 +44,8 @@
 //   codec_math_check order           xcd_contiguous_item (work_order.h) is a
 //                                    bijection on 0 .. n-1 for every n up to
 //                                    4096 and for the bench grids
+//   codec_math_check deal            dealt_item (work_order.h) deals every item once
+//                                    and items at a period evenly
 // Prints "<checked> <failures>" and exits non-zero on any failure.
 #include <math.h>
 #include <stdint.h>
@@ -382,6 +384,37 @@ void check_order() {
   }
 }
 
+// dealt_item over `items` and `blocks` workgroups: every item once (one check),
+// and for every period to 1,024 no workgroup more than `most` even shares of the
+// items at that period (one check a period).
+void check_deal(uint64_t items, uint64_t blocks, uint64_t most) {
+  std::vector<uint32_t> owner(items, ~0u);
+  const uint64_t turns = (items + blocks - 1) / blocks;
+  bool ok = true;
+  for (uint64_t b = 0; b < blocks; ++b) {
+    for (uint64_t turn = 0; turn < turns; ++turn) {
+      const uint64_t item = gdn::dealt_item(b, turn, blocks);
+      if (item >= items) continue;
+      ok = ok && owner[item] == ~0u;
+      owner[item] = static_cast<uint32_t>(b);
+    }
+  }
+  for (uint64_t i = 0; i < items; ++i) ok = ok && owner[i] != ~0u;
+  ++checked;
+  if (!ok) ++failures;
+  for (uint64_t period = 2; period <= 1024; ++period) {
+    ok = true;
+    for (uint64_t offset : {uint64_t{0}, period / 3, period - 1}) {
+      std::vector<uint64_t> load(blocks, 0);
+      uint64_t count = 0;
+      for (uint64_t i = offset; i < items; i += period, ++count) ++load[owner[i]];
+      for (uint64_t l : load) ok = ok && l <= most * ((count + blocks - 1) / blocks);
+    }
+    ++checked;
+    if (!ok) ++failures;
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -407,6 +440,12 @@ int main(int argc, char** argv) {
     check_newton();
   } else if (strcmp(argv[1], "order") == 0) {
     check_order();
+  } else if (strcmp(argv[1], "deal") == 0) {
+    check_deal(960, 256, 3);
+    check_deal(8192, 256, 7);
+    check_deal(61440, 256, 11);
+    for (uint64_t n : {1, 2, 255, 256}) check_deal(n, n, 1);
+    check_deal(257, 256, 2);
   } else {
     return 2;
   }

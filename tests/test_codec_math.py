@@ -116,3 +116,11 @@ def test_xcd_contiguous_order_is_a_bijection(checker):
     every tile exactly once for every grid size up to 4,096 and the bench's."""
     rc, checked, failures = _run(checker, "order")
     assert checked == 4096 + 7 and failures == 0 and rc == 0
+
+
+def test_dealt_items_are_dealt_once_and_evenly(checker):
+    """The Jacobi kernel's workgroup -> head order (csrc/work_order.h): every
+    head once, and heads at any one period spread over the workgroups (in plain
+    strides, the same head of every layer came to 8 of 256 workgroups)."""
+    rc, checked, failures = _run(checker, "deal")
+    assert checked == 8 * 1024 and failures == 0 and rc == 0
