@@ -56,9 +56,17 @@ static_assert(content_bytes(0) + kDigestChars == 21688, "capsule size");
 static_assert(content_bytes(0) % 64 == 56, "the digest tail spans two blocks");
 
 constexpr int kThreads = 256;
-constexpr int kDigestCapsules = 32;  // per digest workgroup, two lanes each
-constexpr int kDigestLanes = 2 * kDigestCapsules;
-constexpr int kDigestThreads = 2 * kDigestLanes;  // producer + consumer wavefront
+constexpr int kDigestCapsules = 32;  // per pair of wavefronts, two lanes each
+constexpr int kDigestPairs = 2;      // most pairs per workgroup
+constexpr int kPairThreads = 2 * 64;  // producer and consumer
+// A workgroup is one pair up to this many capsules (a workgroup per CU), two
+// above.  The wavefronts of two one-pair workgroups on a CU meet on the same two
+// SIMDs; a workgroup of two pairs takes all four, and 16,384 capsules, the most
+// a call admits, are one such workgroup per CU.  Serialize and restore, one /
+// two pairs, us: 3,000 capsules 2,362 / 2,455, 4,096 2,387 / 2,517, 8,192
+// 2,372 / 2,442, 12,288 3,813 / 2,436, 16,384 3,831 / 2,513 (with a lane per
+// capsule 2,944, 2,967, 2,991, 3,042 and 3,111).
+constexpr uint32_t kOnePairCapsules = 256 * kDigestCapsules;
 
 // The expected / written identity, as kernel-argument words.
 struct Identity {
@@ -101,10 +109,6 @@ __device__ __forceinline__ uint32_t xor3(uint32_t x, uint32_t y, uint32_t z) {
 __device__ __forceinline__ uint32_t choose(uint32_t x, uint32_t y, uint32_t z) {
   return __builtin_amdgcn_bitop3_b32(x, y, z, 0xCA);  // (x & y) ^ (~x & z)
 }
-__device__ __forceinline__ uint32_t majority(uint32_t x, uint32_t y, uint32_t z) {
-  return __builtin_amdgcn_bitop3_b32(x, y, z, 0xE8);  // (x&y) ^ (x&z) ^ (y&z)
-}
-
 // x where mask is 0, ~(x ^ y) where it is all ones.
 __device__ __forceinline__ uint32_t same_where(uint32_t x, uint32_t y, uint32_t mask) {
   return __builtin_amdgcn_bitop3_b32(x, y, mask, 0xD2);
@@ -188,13 +192,13 @@ struct DigestArgs {
   uint32_t states;
 };
 
-// One workgroup hashes 32 capsules, two lanes each, with two wavefronts: the
-// producer loads each 64-byte block, expands the message schedule and writes
-// K[t] + W[t] for the block's 64 rounds to a double-buffered LDS ring; the
-// consumer runs only the round function from the ring (section 6.2.2).  One
-// barrier per block: the producer fills slot b + 1 while the consumer works on
-// slot b, and a slot is refilled only after the barrier the consumer reaches
-// when done with it.
+// A pair of wavefronts hashes 32 capsules, two lanes each: the producer loads
+// each 64-byte block, expands the message schedule and writes K[t] + W[t] for
+// the block's 64 rounds to a double-buffered LDS ring; the consumer runs only
+// the round function from the ring (section 6.2.2).  One barrier per block: the
+// producer fills slot b + 1 while the consumer works on slot b, and a slot is
+// refilled only after the barrier the consumer reaches when done with it.  A
+// workgroup is one or two pairs (kOnePairCapsules says when).
 //
 // A batch's time is its longest capsule's chain (699 blocks of 64 rounds), one
 // wavefront's VALU issue, whatever the number of lanes at work.  A round's two
@@ -205,23 +209,28 @@ struct DigestArgs {
 // Maj(a, b, c) is Ch(~(a ^ b), b, c); the new a is the sum of both halves and
 // the new e that of d and the odd half, so each lane adds what its partner
 // offers (d, or the odd half) to its own half.  4,096 capsules, serialize and
-// restore: 2,943 us with a lane per capsule, 2,424 us so.
+// restore: 2,967 us with a lane per capsule, 2,444 us with the even lanes' m read
+// as zeros from the ring, 2,387 us with it masked.
 //
 // kVerify = false: write the digest of each serialized capsule (lengths[i] = 0
 // marks a state the pack kernel skipped).  kVerify = true: the first checks of
 // Restore (state_capsule.cpp:481-494), status[i] = 0 when they all pass.
 template <bool kVerify>
-__global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestArgs a) {
-  // [slot][round / 4][lane]; the even lanes' words stay 0.
-  __shared__ __align__(16) uint4 ring[2][16][kDigestLanes];
-  const int wave = threadIdx.x >> 6;
+__global__ __launch_bounds__(kDigestPairs* kPairThreads) void capsule_digest_kernel(DigestArgs a) {
+  // [pair][slot][round / 4][capsule]
+  __shared__ __align__(16) uint4 rings[kDigestPairs][2][16][kDigestCapsules];
+  __shared__ uint32_t pair_blocks[kDigestPairs];
+  const int pairs = blockDim.x / kPairThreads;
+  const int pair = threadIdx.x / kPairThreads;
+  const bool producer = (threadIdx.x & 64) == 0;
   const int lane = threadIdx.x & 63;
   const bool odd = (lane & 1) != 0;
-  const uint32_t s = blockIdx.x * kDigestCapsules + (lane >> 1);
+  const int capsule = lane >> 1;  // of the pair's
+  const uint32_t s = (blockIdx.x * pairs + pair) * kDigestCapsules + capsule;
+  auto& ring = rings[pair];
 
   // Per-capsule checks, evaluated identically by both lanes of a capsule and
-  // both wavefronts so that their block counts (and so their barrier counts)
-  // agree.
+  // both wavefronts of a pair.
   uint32_t status = GDN_STATE_CODEC_CAPSULE_OK;
   bool hash = false;
   uint8_t* base = nullptr;
@@ -268,21 +277,23 @@ __global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestAr
     }
   }
   const uint32_t blocks = hash ? message_blocks(content) : 0u;
-  uint32_t wave_blocks = blocks;
+  // The workgroup's longest message, and so every wavefront's barrier count.
+  uint32_t most_blocks = blocks;
 #pragma unroll
   for (int mask = 32; mask >= 1; mask >>= 1) {
-    const uint32_t other = __shfl_xor(wave_blocks, mask);
-    wave_blocks = other > wave_blocks ? other : wave_blocks;
+    const uint32_t other = __shfl_xor(most_blocks, mask);
+    most_blocks = other > most_blocks ? other : most_blocks;
+  }
+  if (producer && lane == 0) pair_blocks[pair] = most_blocks;
+  __syncthreads();
+  for (int p = 0; p < pairs; ++p) {
+    most_blocks = pair_blocks[p] > most_blocks ? pair_blocks[p] : most_blocks;
   }
 
-  if (wave == 0) {
+  if (producer) {
     // ---- producer: message schedule plus round constants ----
     const uint32_t full = content / 64;
     const uint64_t* src = reinterpret_cast<const uint64_t*>(base);
-    if (!odd) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) ring[i >> 4][i & 15][lane] = make_uint4(0, 0, 0, 0);
-    }
     uint64_t next[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) next[i] = 0;
@@ -290,7 +301,7 @@ __global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestAr
 #pragma unroll
       for (int i = 0; i < 8; ++i) next[i] = src[i];
     }
-    for (uint32_t block = 0; block < wave_blocks; ++block) {
+    for (uint32_t block = 0; block < most_blocks; ++block) {
       if (odd && block < blocks) {
         uint32_t w[16];
         message_block(base, content, block, next, w);
@@ -316,7 +327,8 @@ __global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestAr
           }
           group[t & 3] = kRound[t] + wt;
           if ((t & 3) == 3) {
-            slot[(t >> 2) * kDigestLanes + lane] = make_uint4(group[0], group[1], group[2], group[3]);
+            slot[(t >> 2) * kDigestCapsules + capsule] =
+                make_uint4(group[0], group[1], group[2], group[3]);
           }
         }
       }
@@ -332,16 +344,16 @@ __global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestAr
   const uint32_t r0 = odd ? 6 : 2, r1 = odd ? 11 : 13, r2 = odd ? 25 : 22;
   const uint32_t odd_mask = odd ? ~0u : 0u;
   const uint32_t even_mask = ~odd_mask;
-  for (uint32_t block = 0; block < wave_blocks; ++block) {
+  for (uint32_t block = 0; block < most_blocks; ++block) {
     __syncthreads();  // slot (block & 1) is ready
     if (block < blocks) {
       const uint4* slot = &ring[block & 1][0][0];
       uint32_t x0 = h[0], x1 = h[1], x2 = h[2], x3 = h[3];
-      uint4 kw = slot[lane];
-      uint32_t m = (x3 & odd_mask) + kw.x;
+      uint4 kw = slot[capsule];
+      uint32_t m = (x3 + kw.x) & odd_mask;
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
-        const uint4 following = slot[(q < 15 ? q + 1 : q) * kDigestLanes + lane];
+        const uint4 following = slot[(q < 15 ? q + 1 : q) * kDigestCapsules + capsule];
         const uint32_t next[4] = {kw.y, kw.z, kw.w, following.x};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -352,7 +364,7 @@ __global__ __launch_bounds__(kDigestThreads) void capsule_digest_kernel(DigestAr
           // read, which must wait two instructions for it; opaque, so that its
           // terms are not added into the chain instead.
           __builtin_amdgcn_sched_barrier(0);
-          m = (x2 & odd_mask) + next[i];
+          m = (x2 + next[i]) & odd_mask;
           asm("" : "+v"(m));
           __builtin_amdgcn_sched_barrier(0);
           x3 = x2;
@@ -894,8 +906,12 @@ bool make_identity(const char* geometry, uint64_t generation, uint64_t epoch, Id
   return true;
 }
 
-uint32_t digest_blocks(uint32_t states) { 
-  return (states + kDigestCapsules - 1) / kDigestCapsules;
+template <bool kVerify>
+int32_t launch_digest(void* stream, const DigestArgs& args) {
+  const uint32_t pairs = args.states <= kOnePairCapsules ? 1 : kDigestPairs;
+  const uint32_t each = pairs * kDigestCapsules;
+  return launch(capsule_digest_kernel<kVerify>, dim3((args.states + each - 1) / each),
+                dim3(pairs * kPairThreads), stream, args);
 }
 
 }  // namespace
@@ -944,8 +960,7 @@ extern "C" int32_t statecentric_gdn_state_codec_capsule_serialize_launch_v1(
                                stream, args);
   if (status != gdn::kStatusOk) return status;
   const gdn::DigestArgs digest{capsules, offsets, lengths, capacity, nullptr, states};
-  return gdn::launch(gdn::capsule_digest_kernel<false>, dim3(gdn::digest_blocks(states)),
-                     dim3(gdn::kDigestThreads), stream, digest);
+  return gdn::launch_digest<false>(stream, digest);
 }
 
 extern "C" int32_t statecentric_gdn_state_codec_capsule_restore_launch_v1(
@@ -969,9 +984,7 @@ extern "C" int32_t statecentric_gdn_state_codec_capsule_restore_launch_v1(
   }
   const gdn::DigestArgs digest{const_cast<uint8_t*>(capsules), offsets, lengths, capacity,
                                status, states};
-  int32_t result = gdn::launch(gdn::capsule_digest_kernel<true>,
-                               dim3(gdn::digest_blocks(states)), dim3(gdn::kDigestThreads),
-                               stream, digest);
+  int32_t result = gdn::launch_digest<true>(stream, digest);
   if (result != gdn::kStatusOk) return result;
   args.capsules = capsules;
   args.offsets = offsets;

@@ -93,7 +93,7 @@ def test_serialize_is_byte_identical_to_the_oracle(device, layout):
 
 @pytest.mark.parametrize("states", [1, 31, 32, 33, 65])
 def test_digests_at_the_edges_of_a_workgroup(device, states):
-    """A digest workgroup takes 32 capsules, two lanes each: batches around
+    """A pair of wavefronts takes 32 capsules, two lanes each: batches around
     that, capsules of unequal length side by side, some skipped or tampered
     with; byte-identical, and restore's digest check fails for exactly the
     tampered ones, whichever half of the digest differs."""
@@ -124,6 +124,49 @@ def test_digests_at_the_edges_of_a_workgroup(device, states):
     fresh = to_device(WG.window_buffers(states, 92, VK), device)
     status = restore_on_gpu(got, offsets, np.array(sizes, np.uint32), positions, fresh, states,
                             VK, device)
+    assert status.tolist() == expect.tolist()
+
+
+@pytest.mark.parametrize("states", [8193, 8250])
+def test_digests_with_two_pairs_of_wavefronts_a_workgroup(device, states):
+    """Above 8,192 capsules a digest workgroup takes 64, two pairs of wavefronts
+    with 32 each, here of unequal lengths (one pair's capsules the shortest, its
+    neighbour's mixed) and with the last pair empty or nearly so: every digest
+    against hashlib, and restore's check fails for exactly the tampered ones."""
+    few = 41
+    print(f"capsule digests, two pairs, states={states}", flush=True)
+    positions = [0 if s // 32 % 2 else (s // 32 + 5 * s) % 16 for s in range(states)]
+    buf = {k: np.ascontiguousarray(np.resize(v, (states,) + v.shape[1:]))
+           for k, v in WG.window_buffers(few, 95, VK, positions=[0] * few).items()}
+    buf["positions"][:, 0] = positions
+    sizes = np.array([C.slot_capsule_bytes(p) for p in positions], np.uint32)
+    offsets = np.concatenate([[0], np.cumsum(sizes[:-1], dtype=np.uint64)]).astype(np.uint64)
+    given = offsets.copy()
+    given[3::777] += np.uint64(4)  # misaligned: not written
+    got, lengths = serialize_on_gpu(to_device(buf, device), states, VK, given, int(sizes.sum()),
+                                    device)
+    written = np.ones(states, bool)
+    written[3::777] = False
+    assert (lengths == np.where(written, sizes, 0)).all()
+    for s in range(states):
+        blob = got[int(offsets[s]):int(offsets[s]) + int(sizes[s])]
+        if written[s]:
+            want = hashlib.sha256(blob[:-64].tobytes()).hexdigest()
+            assert blob[-64:].tobytes().decode() == want, s
+        else:
+            assert (blob == FILL).all(), s
+    for s in (0, 31, 32, 63, 64, 8191, 8192, states - 1):
+        at = int(offsets[s])
+        assert got[at:at + int(sizes[s])].tobytes() == C.slot_serialize(buf, s, VK, IDENTITY), s
+    expect = np.where(written, 0, C.TRUNCATED)
+    checked = np.where(written, sizes, 0).astype(np.uint32)
+    for s in range(1, states, 13):
+        if written[s]:
+            at = int(offsets[s]) + int(sizes[s]) - 64 + (11 * s) % 64
+            got[at] = ord("0") if got[at] != ord("0") else ord("1")
+            expect[s] = C.DIGEST_MISMATCH
+    fresh = to_device(buf, device)
+    status = restore_on_gpu(got, offsets, checked, positions, fresh, states, VK, device)
     assert status.tolist() == expect.tolist()
 
 
