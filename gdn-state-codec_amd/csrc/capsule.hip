@@ -238,9 +238,13 @@ __global__ __launch_bounds__(kDigestPairs* kPairThreads) void capsule_digest_ker
   uint32_t recorded[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) recorded[i] = 0;
-  if (s < a.states) {
-    const uint64_t offset = a.offsets[s];
-    const uint32_t length = a.lengths[s];
+  {
+    // Lanes past the last capsule hash it once more and write nothing: a
+    // wavefront with one quarter of its lanes at work takes 1.5 times as long
+    // (1 to 8 capsules of 699 blocks in a wavefront: 1,490 us, 10 to 32: 1,030).
+    const uint32_t source = min(s, a.states - 1);
+    const uint64_t offset = a.offsets[source];
+    const uint32_t length = a.lengths[source];
     hash = true;
     if constexpr (kVerify) {
       if ((offset & 7u) != 0 || offset > a.capacity || length > a.capacity - offset) {
