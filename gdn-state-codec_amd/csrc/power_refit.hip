@@ -5,8 +5,8 @@
 // For a state whose 16-record window is full, the window's residual operator
 //   R = boundary * S + old compensators * S + sum_j key_j corr_j^T * suffix_j
 // is fitted with four rank-one terms by deflated power iteration (the start
-// vector of rank r is ((r+1)(c+3)) mod 17 - 8, normalized with a 20-step
-// Newton square root), stored as fp16 compensators; R minus the fit is then
+// vector of rank r is ((r+1)(c+3)) mod 17 - 8, normalized with the reference's
+// Newton square root, newton_sqrt), stored as fp16 compensators; R minus the fit is then
 // re-encoded with fresh smoothing sqrt(mean |row|), absmax scales and
 // round-half-away codes, and the window is cleared.
 //
@@ -14,17 +14,16 @@
 // keeps each one on a single thread in the reference's order, so the result is
 // bit-identical to the CPU statement of the reference kernel.
 //
-// One workgroup per state, in two forms (kSplitStates says where the line
-// between them lies):
+// One workgroup per state, in two forms (takes_split_form says which):
 //   split, 256 threads: threads 0..127 own the key rows and 128..255 the value
 //     columns, each with its line's 128 boundary values code / 127 * s * scale
 //     in VGPRs (168, so three states per CU).  An operator application sums on
 //     the side that owns its outputs, while a wavefront of the other side forms
 //     the 24 projections of the compensators, records and fitted ranks.
 //   whole, 128 threads: thread t owns row t and column t, with their codes in
-//     64 VGPRs and the values formed again in every application (eight
-//     instructions a value instead of three), which leaves five states per CU
-//     (31,920 bytes of LDS each).
+//     64 VGPRs and the first 48 of the row's values in 48 more; the other
+//     values are formed again in every application (eight instructions a value
+//     instead of three).  Five states per CU (31,920 bytes of LDS each).
 // In both one wavefront sums a vector's squared norm and normalizes it.  The
 // chains of one state bound the kernel when there are few states (per
 // application 128 products and adds, 24 more terms and 128 adds), VALU issue
@@ -51,21 +50,30 @@ constexpr int kThreads = 128;       // one thread per row (and column)
 constexpr int kSplitThreads = 256;  // one thread per row, one per column
 constexpr int kCodeStride = kDim + 4;
 constexpr float kBoundaryFloor = 1.0e-8f;
-// The split form up to what runs at once with three states per CU: one state's
-// latency is what counts there.  4 iterations, split / whole form (and the
-// form before both, which formed each value from LDS with a rolled loop, a
-// thread for row and column), us: 32 states 158 / 231 (324), 256 states 168 /
-// 241 (298), 768 states 223 / 285 (320), 1,024 states 362 / 306 (325), 8,192
-// states 2,311 / 2,077 (2,288).  At 1,536 and 2,304 states the split form's
-// rounds come out full and it is ahead by 16% and 2%, at 1,280 behind by 7%.
-constexpr uint32_t kSplitStates = 768;
+// The split form up to one round of the chip, and with two iterations or more
+// wherever it takes no more rounds than the whole one, its round being the
+// shorter: from 1,281 to 1,536 states.  Split / whole form with the window's 16
+// steps (before both, with each value formed from LDS by a thread for row and
+// column), us, 4 iterations: 512 states 319 / 377 (427), 768 332 / 387 (432),
+// 800 478 / 399 (439), 1,280 571 / 514 (554), 1,282 580 / 647, 1,408 590 / 660
+// (777), 1,536 598 / 663 (779), 1,792 750 / 760 (837), 2,048 794 / 778 (868),
+// 2,304 876 / 857 (937), 4,096 1,521 / 1,373 (1,567), 8,192 2,876 / 2,543
+// (2,866).  1,536 states with 1 iteration 429 / 425 (472), with 2 490 / 508, with
+// 16 1,287 / 1,649 (2,006).
+constexpr uint32_t kSplitRound = 3 * 256;
+constexpr uint32_t kWholeRound = 5 * 256;
+constexpr bool takes_split_form(uint32_t states, uint32_t iterations) {
+  return states <= kSplitRound ||
+         (iterations > 1 && (states + kSplitRound - 1) / kSplitRound <=
+                                (states + kWholeRound - 1) / kWholeRound);
+}
 
 // In the form with codes in registers, the values of a row's first columns are
 // held as well: what three wavefronts per SIMD leave of the registers.  Such a
 // value costs an application three VALU instructions, one formed from its code
-// eight.  8,192 states, 4 iterations, with the
-// window's 16 steps: 2,660 us with none held, 2,555 with 48, 2,606 with 64 and
-// 2,729 with 80, where more values are spilled (11, 19 and 35 VGPRs).
+// eight.  8,192 states, 4 iterations, with the window's 16 steps: 2,660 us with
+// none held, 2,555 with 48, 2,606 with 64 and 2,729 with 80, where more values
+// are spilled (11, 19 and 35 VGPRs).
 constexpr int kHeldCells = 48;
 
 // f(std::integral_constant<int, c>) for c = 0 .. kDim - 1, expanded at compile
@@ -320,142 +328,142 @@ __device__ __forceinline__ void reencode_rows(PowerShared& sh, float (&cell)[kDi
                                               Sink&& sink) {
   const int row = t;
   if (active) {
-  {
-    // The row's operands stay as fp16 pairs (widened where used) and the
-    // window suffix products, the same for every thread, in scalar
-    // registers, leaving the vector registers to the cells.
-    [[maybe_unused]] const float s = sh.smoothing[row];
-    uint32_t ck2[kRank / 2], nk2[kRank / 2], rk2[kWindow / 2];
-    float suffix[kWindow];
+    {
+      // The row's operands stay as fp16 pairs (widened where used) and the
+      // window suffix products, the same for every thread, in scalar
+      // registers, leaving the vector registers to the cells.
+      [[maybe_unused]] const float s = sh.smoothing[row];
+      uint32_t ck2[kRank / 2], nk2[kRank / 2], rk2[kWindow / 2];
+      float suffix[kWindow];
 #pragma unroll
-    for (int i = 0; i < kRank / 2; ++i) {
-      ck2[i] = reinterpret_cast<const uint32_t*>(sh.ck + row * kRank)[i];
-      nk2[i] = reinterpret_cast<const uint32_t*>(sh.nk + row * kRank)[i];
-    }
-#pragma unroll
-    for (int i = 0; i < kWindow / 2; ++i) rk2[i] = reinterpret_cast<const uint32_t*>(sh.rk + row * kWindow)[i];
-#pragma unroll
-    for (int j = 0; j < kWindow; ++j) {
-      suffix[j] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(sh.record_suffix[j])));
-    }
-    // Every compensator and record product is of two fp16 values, exact in
-    // fp32: one v_fma_mix_f32 each (half_product), and the fitted ranks'
-    // `value -= nk * nv` one fma (minus_half_product), the reference's
-    // roundings throughout.
-    const float neg_zero = opaque_negative_zero();
-    const auto half = [](uint32_t pair, int i) { return i & 1 ? pair >> 16 : pair; };
-    // A column's LDS operands; the next column's are read while this one's
-    // cell is evaluated, so their latency overlaps the arithmetic.
-    struct Operands {
-      int code;     // with kFromCodes
-      float scale;  // with kFromCodes
-      uint2 cv, nv;
-      uint4 r0, r1;
-    };
-    const auto fetch = [&](int column) {
-      Operands o;
-      if constexpr (kFromCodes) {
-        o.code = sh.code[column * kCodeStride + row];
-        o.scale = sh.scales[column];
+      for (int i = 0; i < kRank / 2; ++i) {
+        ck2[i] = reinterpret_cast<const uint32_t*>(sh.ck + row * kRank)[i];
+        nk2[i] = reinterpret_cast<const uint32_t*>(sh.nk + row * kRank)[i];
       }
-      o.cv = *reinterpret_cast<const uint2*>(sh.cv + column * kRank);
-      o.nv = *reinterpret_cast<const uint2*>(sh.nv + column * kRank);
-      const uint4* const rc4 = reinterpret_cast<const uint4*>(sh.rc + column * kWindow);
-      o.r0 = rc4[0];
-      o.r1 = rc4[1];
-      return o;
-    };
-    Operands next = fetch(0);
-    each_column([&](auto c) {
-      constexpr int column = decltype(c)::value;
-      // Opaque to the compiler, so the pairs stay packed in registers.
 #pragma unroll
-      for (int i = 0; i < kRank / 2; ++i) asm volatile("" : "+v"(ck2[i]), "+v"(nk2[i]));
-#pragma unroll
-      for (int i = 0; i < kWindow / 2; ++i) asm volatile("" : "+v"(rk2[i]));
-      const Operands o = next;
-      if constexpr (column + 1 < kDim) next = fetch(column + 1);
-      // Issued here, ahead of this column's arithmetic, not sunk to its end.
-      __builtin_amdgcn_sched_barrier(0);
-      // code / 127 by the two-part division (exact for every integer code).
-      float value;
-      if constexpr (kFromCodes) {
-        value = code_value_arith(static_cast<int8_t>(o.code)) * s * o.scale * bs;
-      } else {
-        value = cell[column] * bs;
-      }
-      const uint32_t cvp[kRank / 2] = {o.cv.x, o.cv.y}, nvp[kRank / 2] = {o.nv.x, o.nv.y};
-#pragma unroll
-      for (int r = 0; r < kRank; ++r) {
-        value += half_product(half(ck2[r / 2], r), half(cvp[r / 2], r), neg_zero) * bs;
-        value = minus_half_product(value, half(nk2[r / 2], r), half(nvp[r / 2], r));
-      }
-      const uint32_t rc2[kWindow / 2] = {o.r0.x, o.r0.y, o.r0.z, o.r0.w,
-                                         o.r1.x, o.r1.y, o.r1.z, o.r1.w};
+      for (int i = 0; i < kWindow / 2; ++i) rk2[i] = reinterpret_cast<const uint32_t*>(sh.rk + row * kWindow)[i];
 #pragma unroll
       for (int j = 0; j < kWindow; ++j) {
-        value += half_product(half(rk2[j / 2], j), half(rc2[j / 2], j), neg_zero) * suffix[j];
+        suffix[j] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(sh.record_suffix[j])));
       }
-      cell[column] = value;
-      // One column ahead at a time: the scheduler would otherwise hoist the
-      // LDS reads of many columns ahead of their use.
+      // Every compensator and record product is of two fp16 values, exact in
+      // fp32: one v_fma_mix_f32 each (half_product), and the fitted ranks'
+      // `value -= nk * nv` one fma (minus_half_product), the reference's
+      // roundings throughout.
+      const float neg_zero = opaque_negative_zero();
+      const auto half = [](uint32_t pair, int i) { return i & 1 ? pair >> 16 : pair; };
+      // A column's LDS operands; the next column's are read while this one's
+      // cell is evaluated, so their latency overlaps the arithmetic.
+      struct Operands {
+        int code;     // with kFromCodes
+        float scale;  // with kFromCodes
+        uint2 cv, nv;
+        uint4 r0, r1;
+      };
+      const auto fetch = [&](int column) {
+        Operands o;
+        if constexpr (kFromCodes) {
+          o.code = sh.code[column * kCodeStride + row];
+          o.scale = sh.scales[column];
+        }
+        o.cv = *reinterpret_cast<const uint2*>(sh.cv + column * kRank);
+        o.nv = *reinterpret_cast<const uint2*>(sh.nv + column * kRank);
+        const uint4* const rc4 = reinterpret_cast<const uint4*>(sh.rc + column * kWindow);
+        o.r0 = rc4[0];
+        o.r1 = rc4[1];
+        return o;
+      };
+      Operands next = fetch(0);
+      each_column([&](auto c) {
+        constexpr int column = decltype(c)::value;
+        // Opaque to the compiler, so the pairs stay packed in registers.
+#pragma unroll
+        for (int i = 0; i < kRank / 2; ++i) asm volatile("" : "+v"(ck2[i]), "+v"(nk2[i]));
+#pragma unroll
+        for (int i = 0; i < kWindow / 2; ++i) asm volatile("" : "+v"(rk2[i]));
+        const Operands o = next;
+        if constexpr (column + 1 < kDim) next = fetch(column + 1);
+        // Issued here, ahead of this column's arithmetic, not sunk to its end.
+        __builtin_amdgcn_sched_barrier(0);
+        // code / 127 by the two-part division (exact for every integer code).
+        float value;
+        if constexpr (kFromCodes) {
+          value = code_value_arith(static_cast<int8_t>(o.code)) * s * o.scale * bs;
+        } else {
+          value = cell[column] * bs;
+        }
+        const uint32_t cvp[kRank / 2] = {o.cv.x, o.cv.y}, nvp[kRank / 2] = {o.nv.x, o.nv.y};
+#pragma unroll
+        for (int r = 0; r < kRank; ++r) {
+          value += half_product(half(ck2[r / 2], r), half(cvp[r / 2], r), neg_zero) * bs;
+          value = minus_half_product(value, half(nk2[r / 2], r), half(nvp[r / 2], r));
+        }
+        const uint32_t rc2[kWindow / 2] = {o.r0.x, o.r0.y, o.r0.z, o.r0.w,
+                                           o.r1.x, o.r1.y, o.r1.z, o.r1.w};
+#pragma unroll
+        for (int j = 0; j < kWindow; ++j) {
+          value += half_product(half(rk2[j / 2], j), half(rc2[j / 2], j), neg_zero) * suffix[j];
+        }
+        cell[column] = value;
+        // One column ahead at a time: the scheduler would otherwise hoist the
+        // LDS reads of many columns ahead of their use.
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    }
+    {
+      float4* const work = reinterpret_cast<float4*>(workspace + row * kDim);
+#pragma unroll
+      for (int q = 0; q < kDim / 4; ++q) {
+        work[q] = make_float4(cell[4 * q], cell[4 * q + 1], cell[4 * q + 2], cell[4 * q + 3]);
+      }
+    }
+
+    // ---- fresh smoothing (row t): sequential sum of |cell| over the columns ----
+    float s_new;
+    {
+      float mean_absolute = 0.0f;
+      each_column([&](auto c) { mean_absolute += fabsf(cell[decltype(c)::value]); });
+      const float mean = mean_absolute / 128.0f;
+      s_new = newton_sqrt(mean > kBoundaryFloor ? mean : kBoundaryFloor);
+      next_smoothing[row] = s_new;
+    }
+    // From here on cell[] holds m = cell / s_new (the cells themselves are in the
+    // workspace already): the scale pass divides once and stores m in place.
+
+    // ---- scales: max over rows of |cell / s| per column -------------------------
+    // The reference keeps `value > maximum ? value : maximum` from 0 over the
+    // rows, which skips NaNs; fmaxf(|m|, 0) maps a NaN to 0 and leaves every
+    // other |m| alone, and a maximum of those is exact in any order.  Each
+    // wavefront reduces its 64 rows with quarter-width reduce-scatters (32
+    // columns across 64 lanes: lane L ends with column L % 32), then the two
+    // wavefronts' maxima meet in LDS.
+    const int lane = t & 63;
+    const int wave = t >> 6;
+#pragma unroll
+    for (int quarter = 0; quarter < 4; ++quarter) {
+#pragma unroll
+      for (int i = 0; i < 32; ++i) cell[32 * quarter + i] = cell[32 * quarter + i] / s_new;
+      const auto magnitude = [&](int i) { return fmaxf(fabsf(cell[32 * quarter + i]), 0.0f); };
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float lo = fold_max<16>(magnitude(i), magnitude(16 + i), lane);
+        const float hi = fold_max<16>(magnitude(8 + i), magnitude(24 + i), lane);
+        v[i] = fold_max<8>(lo, hi, lane);
+        if (i % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = fold_max<4>(v[i], v[i + 4], lane);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) v[i] = fold_max<2>(v[i], v[i + 2], lane);
+      v[0] = fold_max<1>(v[0], v[1], lane);
+      v[0] = max_partner<32>(v[0]);
+      if (lane < 32) {
+        (wave == 0 ? sh.left : sh.right)[32 * quarter + lane] = v[0];
+      }
       __builtin_amdgcn_sched_barrier(0);
-    });
-  }
-  {
-    float4* const work = reinterpret_cast<float4*>(workspace + row * kDim);
-#pragma unroll
-    for (int q = 0; q < kDim / 4; ++q) {
-      work[q] = make_float4(cell[4 * q], cell[4 * q + 1], cell[4 * q + 2], cell[4 * q + 3]);
     }
   }
-
-  // ---- fresh smoothing (row t): sequential sum of |cell| over the columns ----
-  float s_new;
-  {
-    float mean_absolute = 0.0f;
-    each_column([&](auto c) { mean_absolute += fabsf(cell[decltype(c)::value]); });
-    const float mean = mean_absolute / 128.0f;
-    s_new = newton_sqrt(mean > kBoundaryFloor ? mean : kBoundaryFloor);
-    next_smoothing[row] = s_new;
-  }
-  // From here on cell[] holds m = cell / s_new (the cells themselves are in the
-  // workspace already): the scale pass divides once and stores m in place.
-
-  // ---- scales: max over rows of |cell / s| per column -------------------------
-  // The reference keeps `value > maximum ? value : maximum` from 0 over the
-  // rows, which skips NaNs; fmaxf(|m|, 0) maps a NaN to 0 and leaves every
-  // other |m| alone, and a maximum of those is exact in any order.  Each
-  // wavefront reduces its 64 rows with quarter-width reduce-scatters (32
-  // columns across 64 lanes: lane L ends with column L % 32), then the two
-  // wavefronts' maxima meet in LDS.
-  const int lane = t & 63;
-  const int wave = t >> 6;
-#pragma unroll
-  for (int quarter = 0; quarter < 4; ++quarter) {
-#pragma unroll
-    for (int i = 0; i < 32; ++i) cell[32 * quarter + i] = cell[32 * quarter + i] / s_new;
-    const auto magnitude = [&](int i) { return fmaxf(fabsf(cell[32 * quarter + i]), 0.0f); };
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float lo = fold_max<16>(magnitude(i), magnitude(16 + i), lane);
-      const float hi = fold_max<16>(magnitude(8 + i), magnitude(24 + i), lane);
-      v[i] = fold_max<8>(lo, hi, lane);
-      if (i % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = fold_max<4>(v[i], v[i + 4], lane);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) v[i] = fold_max<2>(v[i], v[i + 2], lane);
-    v[0] = fold_max<1>(v[0], v[1], lane);
-    v[0] = max_partner<32>(v[0]);
-    if (lane < 32) {
-      (wave == 0 ? sh.left : sh.right)[32 * quarter + lane] = v[0];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  }  // active
   __syncthreads();  // both wavefronts' column maxima; every cell has been evaluated
   if (active) {
     // Thread t's own slots: no other thread reads them before the barrier.
@@ -835,7 +843,7 @@ int32_t launch_power_refit(void* stream, const int8_t* residual, const float* sm
                        next_scales, next_comp_keys, next_comp_values, residual_workspace,
                        power_iterations};
   void* pointers[] = {const_cast<PowerArgs*>(&args)};
-  const bool split = states <= kSplitStates;
+  const bool split = takes_split_form(states, power_iterations);
   const hipError_t status = hipLaunchKernel(
       split ? reinterpret_cast<const void*>(power_refit_kernel<true>)
             : reinterpret_cast<const void*>(power_refit_kernel<false>),

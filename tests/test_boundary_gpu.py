@@ -298,13 +298,15 @@ def test_quant_only_refit_at_fp16_ties(device):
     assert_same(from_device(d, buf), ref, buf.keys())
 
 
-def test_power_refit_forms_agree_at_their_line(device):
-    """768 states take the split form of the power refit, 769 the whole one:
-    the states they share come out bit for bit the same, among them windows
-    whose first normalization fails (all zero), whose norms lie above 2^32 or
-    below 2^-32 (the root's 20 steps) and whose compensators dominate.  Every
-    128th state and the planted ones against the oracle."""
-    states = 769
+@pytest.mark.parametrize("states", [769, 1281, 1537])
+def test_power_refit_forms_agree_at_their_line(device, states):
+    """768 states take the split form of the power refit, 769 the whole one,
+    as do 1,280; with two iterations or more 1,281 to 1,536 take the split one
+    and 1,537 the whole one again: the states the two share come out bit for
+    bit the same, among them windows whose first normalization fails (all
+    zero), whose norms lie above 2^32 or below 2^-32 (the root's 20 steps) and
+    whose compensators dominate.  Every 128th state and the planted ones
+    against the oracle."""
     from test_boundary_oracle import planted_window
 
     few = planted_window(32, 91)
@@ -332,14 +334,14 @@ def test_power_refit_forms_agree_at_their_line(device):
             stream(), *window_ptrs(d), *out_ptrs(do), dw.data_ptr(), count, 3) == 0
         torch.cuda.synchronize()
         results.append((from_device(do, out), from_device(d, part), dw.cpu().numpy()))
-    (whole, whole_buf, whole_ws), (split, split_buf, split_ws) = results
+    (more, more_buf, more_ws), (fewer, fewer_buf, fewer_ws) = results
     first = np.arange(states - 1)
-    assert_same(_subset(whole, first), split, OUT_NAMES)
-    assert_same(_subset(whole_buf, first), split_buf, buf.keys())
-    assert whole_ws[:-1].tobytes() == split_ws.tobytes()
+    assert_same(_subset(more, first), fewer, OUT_NAMES)
+    assert_same(_subset(more_buf, first), fewer_buf, buf.keys())
+    assert more_ws[:-1].tobytes() == fewer_ws.tobytes()
     idx = np.unique(np.r_[np.arange(0, 16), np.arange(0, states, 128), states - 1])
     ref, ref_out = _subset(buf, idx), _subset(sentinel_outputs(states), idx)
     ref_ws = np.full((idx.size, 128, 128), 7.0, np.float32)
     W.window_boundary_power(ref, ref_out, ref_ws, 3)
-    assert_same(_subset(whole, idx), ref_out, OUT_NAMES)
-    assert whole_ws[idx].tobytes() == ref_ws.tobytes()
+    assert_same(_subset(more, idx), ref_out, OUT_NAMES)
+    assert more_ws[idx].tobytes() == ref_ws.tobytes()
