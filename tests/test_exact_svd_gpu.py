@@ -170,9 +170,10 @@ def test_sweep_limit_flags_unconverged_heads(device):
 
 
 def mixed_heads(count, seed):
-    """Heads for both forms of the SVD in one batch: plain heads, a fourth
-    singular value just above and just below 2^-10 of the first (the direct
-    form's limit), ranks 1 to 5, and four equal leading singular values."""
+    """Heads of one and of several passes in one batch: plain heads, a fourth
+    singular value just above and just below 2^-10 of the first (a pass's
+    limit), ranks 1 to 5, and four leading singular values equal but for the
+    rounding to fp32."""
     g = np.random.default_rng(seed)
     rest = np.linspace(0.9, 0.01, 124)
     out = []
@@ -195,10 +196,9 @@ def mixed_heads(count, seed):
 
 @pytest.mark.parametrize("count", [1, 3, 40, 521])
 def test_direct_and_jacobi_forms_share_a_batch(device, count):
-    """Every head of a mixed batch, whichever form served it, holds the rank-4
-    product to the tolerance of the other tests; 521 heads leave more pending
-    heads than one Jacobi workgroup per CU, none of whose neighbours they may
-    disturb."""
+    """Every head of a mixed batch, whatever passes it took, holds the rank-4
+    product to the tolerance of the other tests, and agrees with the Jacobi
+    form's."""
     dense = mixed_heads(count, 500)
     print(f"exact SVD initializer, mixed batch of {count}", flush=True)
     _, got = run(dense)
@@ -307,6 +307,29 @@ def test_heads_of_few_rows_or_columns(device):
     for a in got:
         assert np.isfinite(a.view(np.float16) if a.dtype == np.uint16 else a).all()
     check_heads(dense, got, rank_deficient=range(len(dense)))
+
+
+@pytest.mark.parametrize("count", [2, 97, 700])
+def test_heads_left_to_jacobi_share_a_batch(device, count):
+    """Every second head a scaled permutation matrix, which the direct form
+    leaves to the Jacobi kernel (350 of 700 heads, more than its 256
+    workgroups): each keeps four of the 128 equal triplets, and the heads
+    between come out with the bytes they have alone."""
+    g = np.random.default_rng(930)
+    dense = datagen.c1_heads(count, 931)
+    for h in range(1, count, 2):
+        dense[h] = np.float32(2.0 ** (h % 7 - 3)) * np.eye(128, dtype=np.float32)[g.permutation(128)]
+    print(f"exact SVD initializer, heads left to Jacobi, heads={count}", flush=True)
+    provider, got = run(dense)
+    assert (got[6] == 0).all()
+    p = host(provider)
+    for h in range(1, count, 2):
+        size = np.abs(p[h]).max()
+        left = np.sort(np.linalg.svd(got[5][h].astype(np.float64), compute_uv=False)) / size
+        assert np.abs(left[:4]).max() <= 1e-6 and np.abs(left[4:] - 1.0).max() <= 1e-6, h
+    _, alone = run(dense[::2])
+    for a, b in zip(got, alone):
+        assert np.ascontiguousarray(a[::2]).tobytes() == b.tobytes()
 
 
 def test_residual_may_overwrite_the_provider_state(device):
