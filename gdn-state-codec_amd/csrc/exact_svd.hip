@@ -374,8 +374,8 @@ __global__ __launch_bounds__(kSvdThreads) void exact_svd_jacobi_kernel(SvdArgs a
 // fp64 MFMA leaves it in; a row's sum is finished inside one 16-lane DPP row
 // and the only traffic through LDS is the vector u and the product G u.  Two
 // heads share a CU (256 VGPRs, under 80 KiB of LDS).  Jacobi -> this form:
-// 32 heads 2.35 -> 0.20 ms, 960 heads 9.2 -> 0.52 ms, 8,192 heads 72.7 -> 3.69
-// ms; 32 heads of rank three (two passes) 0.40 ms.
+// 32 heads 2.35 -> 0.20 ms, 960 heads 9.2 -> 0.52 ms, 8,192 heads 72.7 -> 3.71
+// ms; 32 heads of rank three (two passes) 3.09 -> 0.39 ms.
 //
 // Squaring P costs accuracy only where a singular value is far below the
 // first: its vector's error is about 2^-52 (sigma_1 / sigma_r)^2.  A pass
@@ -383,12 +383,12 @@ __global__ __launch_bounds__(kSvdThreads) void exact_svd_jacobi_kernel(SvdArgs a
 // 2^-10 sigma_1).  A head with fewer than four of them (a state of fewer than
 // four tokens has that rank) takes another pass over what is left of P without
 // the triplets found, which the Gram matrix forms in double from P itself (2^-53
-// of sigma_1 is lost, as in any double form; nothing is kept in fewer bits).  A
-// second pass costs as much as the first.  Where vectors lean on each other
-// (repeated eigenvalues), those up to the first that does are kept and another
-// pass finds the rest: at most four passes, 0.2 ms each for 32 heads, where the
-// Jacobi kernel takes about 2 ms.  A head whose first vector's residual is not
-// at rounding level is marked pending for that kernel.
+// of sigma_1 is lost, as in any double form; nothing is kept in fewer bits); it
+// costs as much as the first.  Where vectors lean on each other (repeated
+// eigenvalues), those up to the first that does are kept and another pass finds
+// the rest: at most four passes, 0.2 ms each for 32 heads, where the Jacobi
+// kernel takes about 2 ms.  A head whose first vector's residual is not at
+// rounding level is marked pending for that kernel.
 constexpr int kDirectThreads = 256;
 constexpr int kStageStride = kDim + 4;                    // floats
 constexpr int kVectorStride = 10;                         // doubles: 16 rows of 8, bank-spread

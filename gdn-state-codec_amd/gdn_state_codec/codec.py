@@ -117,7 +117,8 @@ def exact_svd_boundary(provider: torch.Tensor, check: bool = True, residual=None
     (``GdnStateCodecRuntime._encode_dense_boundary``,
     ``src/gdn_state_codec/runtime.py:335-389``) for fp32 [...,128,128]
     provider heads ([value][key], the dense state transposed): the rank-4
-    truncated SVD of each dense head on the GPU, then the quant-only encode of the fitted residual in the provider layout.
+    truncated SVD of each dense head on the GPU, then the quant-only encode of
+    the fitted residual in the provider layout.
 
     Returns ``(codes, smoothing, scales, compensator_keys, compensator_values,
     residual, status)``: codes int8 [...,value,key], fp16 compensators
