@@ -121,8 +121,8 @@ int32_t statecentric_gdn_state_codec_quantize_boundary_launch_v1(
  * GdnStateCodecRuntime._encode_dense_boundary(dense, "exact_svd")
  * (src/gdn_state_codec/runtime.py:335-389), which calls torch.linalg.svd:
  * the rank-4 truncated SVD of each dense head D = U S V^T (the four largest
- * eigenpairs of D^T D; one-sided Jacobi for a head whose pairs do not come out
- * at rounding level),
+ * eigenpairs of D^T D; one-sided Jacobi for a head whose rows are orthogonal to
+ * begin with or whose pairs do not come out at rounding level),
  * compensator_keys fp16 [heads][128 key][4] = U[:, r] * S[r] and
  * compensator_values fp16 [heads][128 value][4] = V[:, r], r = 0..3 by
  * decreasing singular value; residual fp32 [heads][value][key] = the provider
